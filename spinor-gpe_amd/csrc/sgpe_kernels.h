@@ -51,67 +51,101 @@ template <typename R> __device__ __forceinline__ void quadrant_fix(int q, R sr, 
   *c = ((q + 1) & 2) ? -cc : cc;
 }
 
-template <typename R> __device__ __forceinline__ void sc(R x, R* s, R* c);
-template <> __device__ __forceinline__ void sc<double>(double x, double* s, double* c) {
-  int q;
-  const double r = cw_reduce(x, &q);
+// sin and cos for |r| <= pi/4. Double: minimax polynomials (Remez exchange,
+// relative error 3.4e-18 of sin, 5e-20 of cos before rounding; 2^-53-rounding
+// dominates: largest error 7.4e-17 and 9.6e-17, as the Taylor series with four
+// more terms has). Float: Taylor terms through r^9 / r^10.
+__device__ __forceinline__ void sc_poly(double r, double* s, double* c) {
   const double r2 = r * r;
-  double ps = 2.8114572543455206e-15;
-  ps = fma(ps, r2, -7.647163731819816e-13);
-  ps = fma(ps, r2, 1.6059043836821613e-10);
-  ps = fma(ps, r2, -2.505210838544172e-08);
-  ps = fma(ps, r2, 2.7557319223985893e-06);
-  ps = fma(ps, r2, -0.0001984126984126984);
-  ps = fma(ps, r2, 0.008333333333333333);
-  ps = fma(ps, r2, -0.16666666666666666);
-  const double sr = fma(r * r2, ps, r);
-  double pc = -1.5619206968586225e-16;
-  pc = fma(pc, r2, 4.779477332387385e-14);
-  pc = fma(pc, r2, -1.1470745597729725e-11);
-  pc = fma(pc, r2, 2.08767569878681e-09);
-  pc = fma(pc, r2, -2.755731922398589e-07);
-  pc = fma(pc, r2, 2.48015873015873e-05);
-  pc = fma(pc, r2, -0.001388888888888889);
-  pc = fma(pc, r2, 0.041666666666666664);
+  double ps = 1.5896827972044486e-10;
+  ps = fma(ps, r2, -2.5050758654058057e-08);
+  ps = fma(ps, r2, 2.7557313695231825e-06);
+  ps = fma(ps, r2, -0.00019841269829816967);
+  ps = fma(ps, r2, 0.008333333333322425);
+  ps = fma(ps, r2, -0.16666666666666632);
+  *s = fma(r * r2, ps, r);
+  double pc = -1.1359669918955859e-11;
+  pc = fma(pc, r2, 2.0875723685357163e-09);
+  pc = fma(pc, r2, -2.7557314355247977e-07);
+  pc = fma(pc, r2, 2.4801587289491845e-05);
+  pc = fma(pc, r2, -0.0013888888888874139);
+  pc = fma(pc, r2, 0.0416666666666666);
   pc = fma(pc, r2, -0.5);
-  const double cr = fma(r2, pc, 1.0);
-  quadrant_fix<double>(q, sr, cr, s, c);
+  *c = fma(r2, pc, 1.0);
 }
-template <> __device__ __forceinline__ void sc<float>(float x, float* s, float* c) {
-  // The reduction runs in double for every argument (exact for any float
-  // x): a single-precision reduction for small arguments with the double one
-  // as a fallback put two branches around every sin/cos, and the blocks they
-  // cut the pointwise code into kept its independent sin/cos chains from
-  // overlapping (the complex64 real-time row pass took 0.3 us longer).
-  int q;
-  const float r = (float)cw_reduce((double)x, &q);
+__device__ __forceinline__ void sc_poly(float r, float* s, float* c) {
   const float r2 = r * r;
   float ps = 2.7557319223985893e-06f;
   ps = fmaf(ps, r2, -0.0001984126984126984f);
   ps = fmaf(ps, r2, 0.008333333333333333f);
   ps = fmaf(ps, r2, -0.16666666666666666f);
-  const float sr = fmaf(r * r2, ps, r);
+  *s = fmaf(r * r2, ps, r);
   float pc = -2.755731922398589e-07f;
   pc = fmaf(pc, r2, 2.48015873015873e-05f);
   pc = fmaf(pc, r2, -0.001388888888888889f);
   pc = fmaf(pc, r2, 0.041666666666666664f);
   pc = fmaf(pc, r2, -0.5f);
-  const float cr = fmaf(r2, pc, 1.0f);
-  quadrant_fix<float>(q, sr, cr, s, c);
+  *c = fmaf(r2, pc, 1.0f);
+}
+
+// The reduction runs in double for every argument, also in complex64 (exact
+// for any float x): a single-precision reduction for small arguments with the
+// double one as a fallback put two branches around every sin/cos, and the
+// blocks they cut the pointwise code into kept its independent sin/cos chains
+// from overlapping (the complex64 real-time row pass took 0.3 us longer).
+template <typename R> __device__ __forceinline__ void sc(R x, R* s, R* c) {
+  int q;
+  R sr, cr;
+  sc_poly((R)cw_reduce((double)x, &q), &sr, &cr);
+  quadrant_fix<R>(q, sr, cr, s, c);
 }
 template <typename R> __device__ __forceinline__ R ex(R x);
 template <> __device__ __forceinline__ double ex<double>(double x) { return exp(x); }
 template <> __device__ __forceinline__ float ex<float>(float x) { return expf(x); }
 
+// exp(x) for |x| <= kSmallExp: minimax polynomial of (exp(x) - 1 - x) / x^2
+// (Remez exchange; relative error 3.4e-18 double, 3.1e-9 float before rounding,
+// largest error after it 1.2e-16 and 6.2e-8). No reduction and no scaling.
+__device__ __forceinline__ double ex_poly(double x) {
+  double p = 2.5117848056977748e-08;
+  p = fma(p, x, 2.7631276855506471e-07);
+  p = fma(p, x, 2.7557216339313716e-06);
+  p = fma(p, x, 2.4801489951255983e-05);
+  p = fma(p, x, 0.0001984126991734402);
+  p = fma(p, x, 0.0013888888947006998);
+  p = fma(p, x, 0.008333333333307221);
+  p = fma(p, x, 0.04166666666651544);
+  p = fma(p, x, 0.166666666666667);
+  p = fma(p, x, 0.5000000000000013);
+  return fma(x, fma(p, x, 1.0), 1.0);
+}
+__device__ __forceinline__ float ex_poly(float x) {
+  float p = 0.0013950489013913796f;
+  p = fmaf(p, x, 0.0083688876559632787f);
+  p = fmaf(p, x, 0.04166620583338496f);
+  p = fmaf(p, x, 0.16666518853794891f);
+  p = fmaf(p, x, 0.5000000095175364f);
+  return fmaf(x, fmaf(p, x, 1.0f), 1.0f);
+}
+
+// Arguments up to these bounds take the polynomials without a reduction
+// (SMALL below): the reduced argument is then x itself and the quadrant 0, so
+// sin and cos come out bit-identical either way.
+constexpr double kSmallAngle = 0.785;
+constexpr double kSmallExp = 0.346;
+
 // exp(-i E Delta) for Delta = dt (real time) or -i dt (imaginary time).
-template <typename R, bool IMAG>
+template <typename R, bool IMAG, bool SMALL = false>
 __device__ __forceinline__ typename Cx<R>::T phase_op(R e_dt) {
   typedef typename Cx<R>::T C;
   if constexpr (IMAG) {
-    return C{ex<R>(-e_dt), (R)0};
+    return C{SMALL ? ex_poly(-e_dt) : ex<R>(-e_dt), (R)0};
   } else {
     R s, c;
-    sc<R>(-e_dt, &s, &c);
+    if constexpr (SMALL)
+      sc_poly(-e_dt, &s, &c);
+    else
+      sc<R>(-e_dt, &s, &c);
     return C{c, s};
   }
 }
@@ -451,96 +485,216 @@ __device__ __forceinline__ void part_sums(const double* part, int nt2, int slot,
   out2[1] = v[1];
 }
 
-// Real-space block of the row pass on this thread's points J0 <= j < J1 of row y, both
-// components: U C P C U with the normalization folded in (tensor_propagator.
-// py:244-267). FAST: separable potential (x and y tables) and no or uniform
-// coupling, which is then always applied (the identity when off) with its
-// e^{-i theta} table (ones in the rotated frame); otherwise dense potentials
-// and coupling arrays where present.
-template <typename R, int N, int E, int T, bool IMAG, bool FAST, int J0 = 0, int J1 = E, typename C>
-__device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const InstDev& P, int dur, int y, int t,
-                                              double lam2, C py0, C py1, const C (&tx0)[E], const C (&tx1)[E],
-                                              const C (&tex)[E]) {
-  const R lam = (R)sqrt(lam2);
-  const R lam2r = (R)lam2;
-  const R cf = (R)P.fft_c;
-  const R guu = (R)P.g_uu, gdd = (R)P.g_dd, gud = (R)P.g_ud;
-  const R hdt = (R)(0.5 * P.dt_sub[dur]);
-  const R dts = (R)P.dt_sub[dur];
-  const int cpl = P.coupling;
-  const R ca = (R)P.c_alpha[dur];
-  const C cb = C{(R)P.c_beta_re[dur], (R)P.c_beta_im[dur]};
-  const double* omd = P.omega_dense;
-  const double* vd0 = P.v_dense[0];
-  const double* vd1 = P.v_dense[1];
+// Real-space block of the row pass, U C P C U with the normalization folded in
+// (tensor_propagator.py:244-267), on this thread's points J0 <= j < J1 of row
+// y, both components. The row passes of batched complex64 plans are bound by
+// the number of vector instructions they issue (four cycles each for a wave,
+// in float as in double), the transforms' about half of them, so this block is
+// written for few:
+//  - Every slot-uniform factor is formed once per row (RowCoef): the interaction
+//    phases take the unnormalized densities, and the normalization and the
+//    forward transform's scale ride in the first coupling factor.
+//  - C = [[a, b e^{-i theta}], [b e^{i theta}, a]] has b imaginary in real time
+//    and real in imaginary time: b e^{-i theta} takes two multiplications, C
+//    three fused operations per output part. (Applying e^{-i theta} to psi_1
+//    on both sides of a theta-free C takes two operations less, but there the
+//    table's rounded modulus multiplies all of psi_1 in every sub-step instead
+//    of the coupled part alone: over 20000 complex64 steps the fidelity with
+//    complex128 fell from 0.97 to 0.93.)
+//  - In imaginary time U and P are real factors.
+//  - Where the phases of all points of a wave are small (they are g n dt / 2:
+//    about 1e-2), their sin/cos or exp is a polynomial alone; one wave-uniform
+//    test chooses the code for the whole block (SMALL). Tested per point, it
+//    would cut the block into pieces that cannot overlap.
+// Row pass before and after (dispatch times, us): 8 x 1024^2 complex64
+// imaginary time 75.5 -> 69.6, 16 x 512^2 complex64 imaginary 38.2 -> 35.6, one
+// 2048^2 complex128 real 86.9 -> 83.1, one 512^2 real 10.7 -> 10.2 (complex128)
+// and 7.9 -> 7.3 (complex64).
+template <typename R> struct RowCoef {
+  bool imag, theta;
+  R kuu, kdd, kud;  // interaction phase of U per unnormalized density
+  R sc;             // normalization x forward transform scale
+  R ca, cb;         // a and b of C (b: its imaginary part in real time)
+  R dts;            // sub-step
+  __device__ __forceinline__ RowCoef(const InstDev& P, int dur, double lam2) {
+    const double h = 0.5 * P.dt_sub[dur] * lam2;
+    imag = P.imag != 0;
+    theta = P.theta_x != nullptr;
+    kuu = (R)(P.g_uu * h);
+    kdd = (R)(P.g_dd * h);
+    kud = (R)(P.g_ud * h);
+    sc = (R)(sqrt(lam2) * P.fft_c);
+    ca = (R)P.c_alpha[dur];
+    cb = (R)(imag ? P.c_beta_re[dur] : P.c_beta_im[dur]);
+    dts = (R)P.dt_sub[dur];
+  }
+};
+
+// (p0, p1) <- [[a, b e], [b conj(e), a]] (p0, p1) with b times i in real time;
+// s = b Re(e), r = b Im(e). NT: e = 1 (r unused). a is close to 1: its product
+// is the one that is not rounded by itself (rounded, p (1 - 1e-7) loses the
+// same part of an ulp at every point of the same mantissa, and the populations
+// of a complex64 run drifted by 2e-8 a sub-step).
+template <bool IMAG, bool NT, typename C, typename R>
+__device__ __forceinline__ void mix(C& p0, C& p1, R a, R s, R r) {
+  C q0, q1;
+  if constexpr (NT) {
+    static_assert(IMAG, "theta-free form: imaginary time");
+    q0 = C{fma(a, p0.x, s * p1.x), fma(a, p0.y, s * p1.y)};
+    q1 = C{fma(a, p1.x, s * p0.x), fma(a, p1.y, s * p0.y)};
+  } else if constexpr (IMAG) {
+    q0 = C{fma(a, p0.x, fma(s, p1.x, -r * p1.y)), fma(a, p0.y, fma(s, p1.y, r * p1.x))};
+    q1 = C{fma(a, p1.x, fma(s, p0.x, r * p0.y)), fma(a, p1.y, fma(s, p0.y, -r * p0.x))};
+  } else {
+    q0 = C{fma(a, p0.x, -fma(s, p1.y, r * p1.x)), fma(a, p0.y, fma(s, p1.x, -r * p1.y))};
+    q1 = C{fma(a, p1.x, fma(-s, p0.y, r * p0.x)), fma(a, p1.y, fma(s, p0.x, r * p0.y))};
+  }
+  p0 = q0;
+  p1 = q1;
+}
+
+// Interaction phases of one point.
+template <typename R, typename C>
+__device__ __forceinline__ void point_phases(C p0, C p1, const RowCoef<R>& k, R* e0, R* e1) {
+  const R m0 = p0.x * p0.x + p0.y * p0.y;
+  const R m1 = p1.x * p1.x + p1.y * p1.y;
+  *e0 = k.kuu * m0 + k.kud * m1;
+  *e1 = k.kdd * m1 + k.kud * m0;
+}
+template <typename R> __device__ __forceinline__ R larger(R a, R b) { return fmax(a, fabs(b)); }
+
+// Code variants of the block. NT: no coupling phase (theta = 0).
+enum { PV_REAL_SMALL, PV_REAL, PV_IMAG_SMALL_NT, PV_IMAG_SMALL, PV_IMAG };
+template <int V> struct PointVariant { static constexpr int v = V; };
+
+// Calls f(PointVariant<V>) for the variant of an instance; `top` is the
+// largest phase of this thread's points. The choice is uniform over the wave.
+template <typename R, class F>
+__device__ __forceinline__ void with_variant(const RowCoef<R>& k, R top, F&& f) {
+  if (k.imag) {
+    if (__builtin_amdgcn_ballot_w64(!(top <= (R)kSmallExp)))
+      f(PointVariant<PV_IMAG>());
+    else if (k.theta)
+      f(PointVariant<PV_IMAG_SMALL>());
+    else
+      f(PointVariant<PV_IMAG_SMALL_NT>());
+  } else if (__builtin_amdgcn_ballot_w64(!(top <= (R)kSmallAngle))) {
+    f(PointVariant<PV_REAL>());
+  } else {
+    f(PointVariant<PV_REAL_SMALL>());
+  }
+}
+
+// One point. FAST: separable potential (x and y tables tx, py) and uniform
+// coupling factors; otherwise `a`, `b` are the point's coupling factors and
+// f0, f1 its potential factors.
+template <typename R, int V, typename C>
+__device__ __forceinline__ void point_ops(C& p0, C& p1, R e0, R e1, R sc, R a, R b, C f0, C f1, C e) {
+  constexpr bool IMAG = V >= PV_IMAG_SMALL_NT;
+  constexpr bool SMALL = V != PV_REAL && V != PV_IMAG;
+  constexpr bool NT = V == PV_IMAG_SMALL_NT;
+  const C u0 = phase_op<R, IMAG, SMALL>(e0);
+  const C u1 = phase_op<R, IMAG, SMALL>(e1);
+  const R s = NT ? b : b * e.x, r = NT ? (R)0 : b * e.y;
+  p0 = mul_phase<IMAG>(p0, u0);
+  p1 = mul_phase<IMAG>(p1, u1);
+  // First half of the coupling (tensor_propagator.py:252-254), scaled.
+  mix<IMAG, NT>(p0, p1, a * sc, s * sc, NT ? (R)0 : r * sc);
+  p0 = mul_phase<IMAG>(p0, f0);       // potential (:256)
+  p1 = mul_phase<IMAG>(p1, f1);
+  mix<IMAG, NT>(p0, p1, a, s, r);     // second half (:258-260)
+  p0 = mul_phase<IMAG>(p0, u0);       // the same U again (:267)
+  p1 = mul_phase<IMAG>(p1, u1);
+}
+
+// x times y factor of a potential phase (real in imaginary time).
+template <bool IMAG, typename C> __device__ __forceinline__ C pot_factor(C tx, C py) {
+  if constexpr (IMAG)
+    return C{tx.x * py.x, 0};
+  else
+    return cmul(tx, py);
+}
+
+// Points J0 <= j < J1 of a row on the fast operator path, in one variant.
+template <typename R, int V, int E, int J0, int J1, typename C>
+__device__ __forceinline__ void fast_points(C (&a0)[E], C (&a1)[E], const RowCoef<R>& k, C py0, C py1,
+                                            const C (&tx0)[E], const C (&tx1)[E], const C (&tex)[E]) {
+  constexpr bool IMAG = V >= PV_IMAG_SMALL_NT;
 #pragma unroll
   for (int j = J0; j < J1; ++j) {
-    const int x = t + j * T;
-    C p0 = a0[j], p1 = a1[j];
-    // Interaction half step U_s = exp(-i (g n) Delta/2) from the normalized
-    // densities (tensor_propagator.py:247-250); U is reused after C P C (:267).
-    const R n0 = lam2r * (p0.x * p0.x + p0.y * p0.y);
-    const R n1 = lam2r * (p1.x * p1.x + p1.y * p1.y);
-    const C u0 = phase_op<R, IMAG>((guu * n0 + gud * n1) * hdt);
-    const C u1 = phase_op<R, IMAG>((gdd * n1 + gud * n0) * hdt);
-    p0 = cscale(mul_phase<IMAG>(p0, u0), lam);
-    p1 = cscale(mul_phase<IMAG>(p1, u1), lam);
-    R alpha = ca;
-    C b01 = cb, b10 = cb;
-    bool apply = true;
-    if constexpr (FAST) {
-      const C e = tex[j];
-      b10 = cmul(b01, cconj(e));
-      b01 = cmul(b01, e);
-    } else {
-      apply = cpl != 0;
-      if (cpl == 2) {
-        const R ang = (R)omd[(size_t)y * N + x] * dts * (R)0.25;
-        if constexpr (IMAG) {
-          const R e = ex<R>(ang), ei = (R)1 / e;
-          alpha = (R)0.5 * (e + ei);
-          b01 = C{(R)-0.5 * (e - ei), (R)0};
-        } else {
-          R s, c;
-          sc<R>(ang, &s, &c);
-          alpha = c;
-          b01 = C{(R)0, -s};
+    R e0, e1;
+    point_phases<R>(a0[j], a1[j], k, &e0, &e1);
+    point_ops<R, V>(a0[j], a1[j], e0, e1, k.sc, k.ca, k.cb, pot_factor<IMAG>(tx0[j], py0),
+                    pot_factor<IMAG>(tx1[j], py1), tex[j]);
+  }
+}
+
+// Largest phase of the points J0 <= j < J1 (fast operator path).
+template <typename R, int E, int J0, int J1, typename C>
+__device__ __forceinline__ R fast_top(const C (&a0)[E], const C (&a1)[E], const RowCoef<R>& k) {
+  R top = (R)0;
+#pragma unroll
+  for (int j = J0; j < J1; ++j) {
+    R e0, e1;
+    point_phases<R>(a0[j], a1[j], k, &e0, &e1);
+    top = larger(larger(top, e0), e1);
+  }
+  return top;
+}
+
+// Points J0 <= j < J1 of a row: FAST as above, else with dense potentials and
+// coupling arrays where the slot has them.
+template <typename R, int N, int E, int T, bool FAST, int J0 = 0, int J1 = E, typename C>
+__device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const InstDev& P, const RowCoef<R>& k, int y,
+                                              int t, C py0, C py1, const C (&tx0)[E], const C (&tx1)[E],
+                                              const C (&tex)[E]) {
+  if constexpr (FAST) {
+    with_variant<R>(k, fast_top<R, E, J0, J1>(a0, a1, k), [&](auto v) {
+      fast_points<R, decltype(v)::v, E, J0, J1>(a0, a1, k, py0, py1, tx0, tx1, tex);
+    });
+  } else {
+    constexpr int M = J1 - J0;
+    const double* vd0 = P.v_dense[0];
+    const double* vd1 = P.v_dense[1];
+    const double* omd = P.coupling == 2 ? P.omega_dense : nullptr;
+    const size_t base = (size_t)y * N + t;
+    R v0[M], v1[M], an[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      const size_t at = base + (J0 + i) * T;
+      v0[i] = vd0 ? (R)ld_global(vd0 + at) * k.dts : (R)0;
+      v1[i] = vd1 ? (R)ld_global(vd1 + at) * k.dts : (R)0;
+      an[i] = omd ? (R)ld_global(omd + at) * k.dts * (R)0.25 : (R)0;
+    }
+    R top = fast_top<R, E, J0, J1>(a0, a1, k);
+#pragma unroll
+    for (int i = 0; i < M; ++i) top = larger(larger(larger(top, v0[i]), v1[i]), an[i]);
+    with_variant<R>(k, top, [&](auto v) {
+      constexpr int V = decltype(v)::v == PV_IMAG_SMALL_NT ? PV_IMAG_SMALL : decltype(v)::v;
+      constexpr bool IMAG = V >= PV_IMAG_SMALL_NT;
+      constexpr bool SMALL = V != PV_REAL && V != PV_IMAG;
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        const int j = J0 + i;
+        R a = k.ca, b = k.cb;
+        if (omd) {
+          if constexpr (IMAG) {
+            const R g = SMALL ? ex_poly(an[i]) : ex<R>(an[i]), gi = (R)1 / g;
+            a = (R)0.5 * (g + gi);
+            b = (R)-0.5 * (g - gi);
+          } else {
+            const C u = phase_op<R, false, SMALL>(an[i]);
+            a = u.x;
+            b = u.y;
+          }
         }
-        b10 = b01;
+        const C f0 = vd0 ? phase_op<R, IMAG, SMALL>(v0[i]) : pot_factor<IMAG>(tx0[j], py0);
+        const C f1 = vd1 ? phase_op<R, IMAG, SMALL>(v1[i]) : pot_factor<IMAG>(tx1[j], py1);
+        R e0, e1;
+        point_phases<R>(a0[j], a1[j], k, &e0, &e1);
+        point_ops<R, V>(a0[j], a1[j], e0, e1, k.sc, a, b, f0, f1, tex[j]);
       }
-      if (cpl) {
-        const C e = tex[j];
-        b10 = cmul(b01, cconj(e));
-        b01 = cmul(b01, e);
-      }
-    }
-    // Coupling half step C (tensor_propagator.py:252-254).
-    if (apply) {
-      const C q0 = cadd(cscale(p0, alpha), cmul(b01, p1));
-      const C q1 = cadd(cmul(b10, p0), cscale(p1, alpha));
-      p0 = q0;
-      p1 = q1;
-    }
-    // Potential step P_s = exp(-i V_s Delta) (tensor_propagator.py:256).
-    C q0, q1;
-    if constexpr (FAST) {
-      q0 = cmul(tx0[j], py0);
-      q1 = cmul(tx1[j], py1);
-    } else {
-      q0 = vd0 ? phase_op<R, IMAG>((R)vd0[(size_t)y * N + x] * dts) : cmul(tx0[j], py0);
-      q1 = vd1 ? phase_op<R, IMAG>((R)vd1[(size_t)y * N + x] * dts) : cmul(tx1[j], py1);
-    }
-    p0 = cmul(p0, q0);
-    p1 = cmul(p1, q1);
-    // Second coupling half step (tensor_propagator.py:258-260).
-    if (apply) {
-      const C s0 = cadd(cscale(p0, alpha), cmul(b01, p1));
-      const C s1 = cadd(cmul(b10, p0), cscale(p1, alpha));
-      p0 = s0;
-      p1 = s1;
-    }
-    a0[j] = cscale(mul_phase<IMAG>(p0, u0), cf);
-    a1[j] = cscale(mul_phase<IMAG>(p1, u1), cf);
+    });
   }
 }
 
@@ -566,19 +720,15 @@ __device__ __forceinline__ void load_x_tables(C (&tx0)[E], C (&tx1)[E], C (&tex)
 // The row pointwise block point by point from point J on, point J's tables
 // already loaded: point J + 1's tables are loaded first, so their latency
 // overlaps point J's arithmetic, and at most two points' tables are live.
-template <typename R, int N, int E, int T, bool FAST, int J, typename C>
-__device__ __forceinline__ void pointwise_points(C (&a0)[E], C (&a1)[E], const InstDev& P, int dur, int y, int t,
-                                                 double lam2, C py0, C py1, C (&tx0)[E], C (&tx1)[E], C (&tex)[E],
-                                                 const C* px0, const C* px1, const C* eth, const C* tws) {
+// `point` is called with std::integral_constant-like PointVariant<J>.
+template <int E, int T, int J, typename C, class F>
+__device__ __forceinline__ void pointwise_points(int t, C (&tx0)[E], C (&tx1)[E], C (&tex)[E], const C* px0,
+                                                 const C* px1, const C* eth, const C* tws, F&& point) {
   if constexpr (J < E) {
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (J + 1 < E) load_x_tables<E, T, J + 1, J + 2>(tx0, tx1, tex, px0, px1, eth, tws, t);
-    if (P.imag)
-      row_pointwise<R, N, E, T, true, FAST, J, J + 1>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex);
-    else
-      row_pointwise<R, N, E, T, false, FAST, J, J + 1>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex);
-    pointwise_points<R, N, E, T, FAST, J + 1>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex, px0, px1, eth,
-                                              tws);
+    point(PointVariant<J>());
+    pointwise_points<E, T, J + 1>(t, tx0, tx1, tex, px0, px1, eth, tws, point);
   }
 }
 
@@ -711,24 +861,36 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   // two 2048-point workgroups share a CU). Complex64 radix >= 8 uses the
   // halves, which already fit 3 waves per SIMD (point by point would only
   // add latency).
+  const RowCoef<R> k(P, dur, lam2);
   if constexpr (E >= 8 && sizeof(C) == 16) {
     load_x_tables<E, T, 0, 1>(tx0, tx1, tex, px0, px1, eth, tws, t);
-    pointwise_points<R, N, E, T, !GENERAL, 0>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex, px0, px1, eth,
-                                              tws);
+    if constexpr (GENERAL)
+      pointwise_points<E, T, 0>(t, tx0, tx1, tex, px0, px1, eth, tws, [&](auto j) {
+        constexpr int J = decltype(j)::v;
+        row_pointwise<R, N, E, T, false, J, J + 1>(a0, a1, P, k, y, t, py0, py1, tx0, tx1, tex);
+      });
+    else {
+      const R top = fast_top<R, E, 0, E>(a0, a1, k);
+      // Opaque copies: the densities are formed again point by point rather
+      // than held for all points at once (32 registers, past 256).
+#pragma unroll
+      for (int j = 0; j < E; ++j)
+        asm volatile("" : "+v"(a0[j].x), "+v"(a0[j].y), "+v"(a1[j].x), "+v"(a1[j].y));
+      with_variant<R>(k, top, [&](auto v) {
+        pointwise_points<E, T, 0>(t, tx0, tx1, tex, px0, px1, eth, tws, [&](auto j) {
+          constexpr int J = decltype(j)::v;
+          fast_points<R, decltype(v)::v, E, J, J + 1>(a0, a1, k, py0, py1, tx0, tx1, tex);
+        });
+      });
+    }
   } else {
     constexpr int H = kEarlyTables ? E : E / 2;
     if constexpr (!kEarlyTables) load_x_tables<E, T, 0, H>(tx0, tx1, tex, px0, px1, eth, tws, t);
-    if (P.imag)
-      row_pointwise<R, N, E, T, true, !GENERAL, 0, H>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex);
-    else
-      row_pointwise<R, N, E, T, false, !GENERAL, 0, H>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex);
+    row_pointwise<R, N, E, T, !GENERAL, 0, H>(a0, a1, P, k, y, t, py0, py1, tx0, tx1, tex);
     if constexpr (H < E) {
       __builtin_amdgcn_sched_barrier(0);
       load_x_tables<E, T, H, E>(tx0, tx1, tex, px0, px1, eth, tws, t);
-      if (P.imag)
-        row_pointwise<R, N, E, T, true, !GENERAL, H, E>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex);
-      else
-        row_pointwise<R, N, E, T, false, !GENERAL, H, E>(a0, a1, P, dur, y, t, lam2, py0, py1, tx0, tx1, tex);
+      row_pointwise<R, N, E, T, !GENERAL, H, E>(a0, a1, P, k, y, t, py0, py1, tx0, tx1, tex);
     }
   }
   // Large rows: the forward transform and the stores index by an opaque copy
@@ -743,7 +905,7 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   // the CUs' slots already, only the recomputation remains (+2 %).
   constexpr size_t kLdsWg = kData * (kDb ? 2 : 1) + (kTw ? (size_t)N * sizeof(C) : 0);
   constexpr int kLdsWaves = (int)(kLdsBytes / kLdsWg) * ((ROWS * T + 63) / 64) / 4;
-  constexpr bool kOpaque = N >= 4096 || (N >= 1024 && kLdsWaves >= 3);
+  constexpr bool kOpaque = N >= 2048 || (N >= 1024 && kLdsWaves >= 3);
   int tf = t;
   if constexpr (kOpaque) asm volatile("" : "+v"(tf));
   // The forward transform starts on the buffer pair the inverse one read
@@ -775,8 +937,19 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   }
 }
 
+// Waves per SIMD asked of the compiler: two for the complex128 radix >= 8 row
+// passes whose LDS admits two (it would otherwise take 260-298 registers for
+// some of them, which leaves one).
+template <typename R, int N, int E, int ROWS> constexpr int row_min_waves() {
+  constexpr size_t cs = sizeof(typename Cx<R>::T);
+  constexpr size_t data = (size_t)ROWS * 2 * N * cs;
+  constexpr size_t lds = data + (tw_in_lds(data, N, cs) ? (size_t)N * cs : 0);
+  constexpr int waves = (int)(kLdsBytes / lds) * ((ROWS * (N / E) + 63) / 64) / 4;
+  return E >= 8 && cs == 16 && waves >= 2 ? 2 : 1;
+}
+
 template <typename R, int N, int E, int ROWS, bool GENERAL>
-__global__ __launch_bounds__(ROWS*(N / E)) void row_pass_kernel(const InstDev* __restrict__ insts,
+__global__ __launch_bounds__(ROWS*(N / E), (row_min_waves<R, N, E, ROWS>())) void row_pass_kernel(const InstDev* __restrict__ insts,
                                                                 RunDev* __restrict__ runs, void* direct_psi,
                                                                 int direct_n,
                                                                 const typename Cx<R>::T* __restrict__ tws,
@@ -920,10 +1093,8 @@ __global__ __launch_bounds__(ROWS * 2 * (N / E)) void row_split_kernel(const Ins
     p0[j] = sm[V::at(tid + j * TP)];
     p1[j] = sm[N + V::at(tid + j * TP)];
   }
-  if (P.imag)
-    row_pointwise<R, N, EP, TP, true, !GENERAL>(p0, p1, P, dur, y, tid, lam2, py0, py1, tx0, tx1, tex);
-  else
-    row_pointwise<R, N, EP, TP, false, !GENERAL>(p0, p1, P, dur, y, tid, lam2, py0, py1, tx0, tx1, tex);
+  const RowCoef<R> k(P, dur, lam2);
+  row_pointwise<R, N, EP, TP, !GENERAL>(p0, p1, P, k, y, tid, py0, py1, tx0, tx1, tex);
 #pragma unroll
   for (int j = 0; j < EP; ++j) {
     sm[V::at(tid + j * TP)] = p0[j];
