@@ -362,8 +362,8 @@ static int ctx_roots(sgpe_ctx* ctx, int prec, int n, const void** out) {
 
 // Dynamic LDS of a kernel with data_bytes of exchange buffers for n-point
 // transforms: the twiddle table joins it when it fits (tw_in_lds), and the
-// column pass adds its `tables` (the 2 kinetic y-tables) when those fit
-// too; the same predicates as in the kernels.
+// column pass adds its `tables` (the kinetic y table) when they fit too; the
+// same predicates as in the kernels.
 static size_t lds_bytes(size_t data_bytes, int n, size_t cs, int tables = 0) {
   size_t total = data_bytes;
   if (tw_in_lds(data_bytes, n, cs)) {
@@ -372,7 +372,7 @@ static size_t lds_bytes(size_t data_bytes, int n, size_t cs, int tables = 0) {
   }
   return std::max<size_t>(total, 256);
 }
-static const int kColTables = 2;
+static const int kColTables = 1;
 
 // Dynamic LDS of a column pass: exchange buffer, tables, and the separate
 // slot for its end-of-pass sums when it fits (col_sum_separate).
@@ -613,7 +613,7 @@ static void launch_row(sgpe_plan* p, hipStream_t s, int dur, int first, hipEvent
 }
 
 static void issue_sub_step(sgpe_plan* p, hipStream_t s, int which, int first) {
-  launch_col(p, s, COL_MID, p->last_dur, which);
+  launch_col(p, s, first ? COL_MID_S : COL_MID, p->last_dur, which);
   launch_row(p, s, which, first);
   p->last_dur = which;
   p->pending = true;
@@ -864,6 +864,7 @@ static int plan_load_slot(sgpe_plan* p, int slot, const sgpe_inst_desc* d, void*
 
   Staging st;
   size_t o_kx[2][2], o_ky[2][2], o_px[2][2], o_py[2][2], o_eth = 0;
+  size_t o_k2x[2][2][2], o_k2y[2][2][2];  // [previous][current duration][component]
   size_t o_tx[2], o_ty[2], o_vx[2], o_vy[2], o_thx = 0, o_td[2], o_vd[2], o_om = 0;
   const size_t dense = (size_t)ny * nx * sizeof(double);
   for (int s = 0; s < 2; ++s) {
@@ -901,9 +902,21 @@ static int plan_load_slot(sgpe_plan* p, int slot, const sgpe_inst_desc* d, void*
   for (int dd = 0; dd < 2; ++dd)
     for (int s = 0; s < 2; ++s) {
       o_kx[dd][s] = o_ky[dd][s] = o_px[dd][s] = o_py[dd][s] = 0;
+      for (int dc = 0; dc < 2; ++dc) o_k2x[dd][dc][s] = o_k2y[dd][dc][s] = 0;
       if (!d->t_dense[s]) {
-        o_kx[dd][s] = st.add(nx * cs);
-        o_ky[dd][s] = st.add(ny * cs);
+        if (!imag) {  // imaginary time reads the pairs alone
+          o_kx[dd][s] = st.add(nx * cs);
+          o_ky[dd][s] = st.add(ny * cs);
+        }
+        for (int dc = 0; dc < 2; ++dc) {
+          if (!imag && dc < dd) {  // one phase of both half steps: symmetric
+            o_k2x[dd][dc][s] = o_k2x[dc][dd][s];
+            o_k2y[dd][dc][s] = o_k2y[dc][dd][s];
+            continue;
+          }
+          o_k2x[dd][dc][s] = st.add(nx * cs);
+          o_k2y[dd][dc][s] = st.add(ny * cs);
+        }
       }
       if (!d->v_dense[s]) {
         o_px[dd][s] = st.add(nx * cs);
@@ -913,21 +926,34 @@ static int plan_load_slot(sgpe_plan* p, int slot, const sgpe_inst_desc* d, void*
   const size_t o_part = st.add((size_t)PART_SLOTS * 2 * nx * sizeof(double));
   const size_t o_epart = st.add((size_t)EPART_SLOTS * (2 * nx + ny) * sizeof(double));
 
-  // Phase tables in float64, rounded once to the plan precision.
+  // Phase tables in float64, rounded once to the plan precision. Kinetic: K of
+  // each sub-step (real time), then the pairs (InstDev::k2x).
+  for (int s = 0; s < 2; ++s) {
+    if (d->t_dense[s]) continue;
+    for (int axis = 0; axis < 2; ++axis) {
+      const double* e = axis ? d->t_y[s] : d->t_x[s];
+      const int n = axis ? ny : nx;
+      for (int i = 0; i < n; ++i) {
+        double re[2], im[2];
+        for (int dd = 0; dd < 2; ++dd) {
+          phase_host(e[i] * (0.5 * dts[dd]), imag, &re[dd], &im[dd]);
+          if (const size_t o = axis ? o_ky[dd][s] : o_kx[dd][s]) put_cplx(st, o, prec, i, re[dd], im[dd]);
+        }
+        for (int dp = 0; dp < 2; ++dp)
+          for (int dc = imag ? 0 : dp; dc < 2; ++dc) {
+            const size_t o = axis ? o_k2y[dp][dc][s] : o_k2x[dp][dc][s];
+            if (imag)
+              put_cplx(st, o, prec, i, re[dp], re[dc]);
+            else
+              put_cplx(st, o, prec, i, re[dp] * re[dc] - im[dp] * im[dc], re[dp] * im[dc] + im[dp] * re[dc]);
+          }
+      }
+    }
+  }
   for (int dd = 0; dd < 2; ++dd) {
     const double dt = dts[dd];
     for (int s = 0; s < 2; ++s) {
       double re, im;
-      if (!d->t_dense[s]) {
-        for (int i = 0; i < nx; ++i) {
-          phase_host(d->t_x[s][i] * (0.5 * dt), imag, &re, &im);
-          put_cplx(st, o_kx[dd][s], prec, i, re, im);
-        }
-        for (int i = 0; i < ny; ++i) {
-          phase_host(d->t_y[s][i] * (0.5 * dt), imag, &re, &im);
-          put_cplx(st, o_ky[dd][s], prec, i, re, im);
-        }
-      }
       if (!d->v_dense[s]) {
         for (int i = 0; i < nx; ++i) {
           phase_host(d->v_x[s][i] * dt, imag, &re, &im);
@@ -984,6 +1010,10 @@ static int plan_load_slot(sgpe_plan* p, int slot, const sgpe_inst_desc* d, void*
     for (int dd = 0; dd < 2; ++dd) {
       h.kx[dd][s] = P(o_kx[dd][s]);
       h.ky[dd][s] = P(o_ky[dd][s]);
+      for (int dc = 0; dc < 2; ++dc) {
+        h.k2x[dd][dc][s] = P(o_k2x[dd][dc][s]);
+        h.k2y[dd][dc][s] = P(o_k2y[dd][dc][s]);
+      }
       h.px[dd][s] = P(o_px[dd][s]);
       h.py[dd][s] = P(o_py[dd][s]);
     }
@@ -1687,7 +1717,7 @@ int sgpe_profile_full_steps(sgpe_plan* p, int n_steps, double* out4) {
     for (int i = 0; i < n_steps; ++i) {
       const int durs[3] = {DUR_OUT, DUR_IN, DUR_OUT};
       for (int j = 0; j < 3; ++j) {
-        launch_col(p, s, COL_MID, p->last_dur, durs[j], ev[2 * k], ev[2 * k + 1]);
+        launch_col(p, s, j == 0 ? COL_MID_S : COL_MID, p->last_dur, durs[j], ev[2 * k], ev[2 * k + 1]);
         ++k;
         launch_row(p, s, durs[j], j == 0, ev[2 * k], ev[2 * k + 1]);
         ++k;

@@ -64,8 +64,9 @@ enum {
 
 // Column-pass modes.
 enum {
-  COL_MID = 0,    // DFT_y, K_prev, [S], K_cur, [NRM], IDFT_y (or entry if FORM_KSPACE)
+  COL_MID = 0,    // DFT_y, K_prev K_cur, [NRM], IDFT_y (or entry if FORM_KSPACE)
   COL_EXIT = 1,   // DFT_y, K_prev, [S]          -> k-space (not normalized)
+  COL_MID_S = 2,  // COL_MID with the sum S between K_prev and K_cur (the first sub-step: populations)
 };
 
 // Per-instance parameters, read-only for kernels (device memory).
@@ -84,6 +85,12 @@ struct InstDev {
   // Kinetic phase K_s = exp(-i T_s Delta/2), separable: kx[d][s][jx] * ky[d][s][jy]
   const void* kx[2][2];
   const void* ky[2][2];
+  // K_prev K_cur of a column pass between sub-steps dp and dc, separable, as
+  // k2x[dp][dc][s][jx], k2y[dp][dc][s][jy]: in real time the phase of both half
+  // steps; in imaginary time, where both factors are real, the pair (K_prev,
+  // K_cur) as real and imaginary part.
+  const void* k2x[2][2][2];
+  const void* k2y[2][2][2];
   const double* t_dense[2];      // non-null: dense T_s (f64, ny*nx), evaluated per pixel
   // Potential phase P_s = exp(-i V_s Delta), separable: px[d][s][jx] * py[d][s][jy]
   const void* px[2][2];

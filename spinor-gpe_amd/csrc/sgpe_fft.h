@@ -419,10 +419,15 @@ __device__ __forceinline__ void block_sum_thread0(double (&v)[NV], double* scrat
 }
 
 // LDS for the column pass's end-of-pass sums (2 doubles per wave, up to 16
-// waves), placed after its exchange buffer and tables when that still fits
-// in LDS (same predicate on host and device); otherwise the sums reuse the
-// exchange buffer (block_sum).
+// waves), placed after its exchange buffer and tables where that does not
+// cost a workgroup per CU (same predicate on host and device); otherwise the
+// sums reuse the exchange buffer (block_sum, two more barriers). Tiles of a
+// power of two fill a CU's 160 KiB exactly at 32 + 8, 64 + 16 or 128 + 32
+// KiB, so the 256 bytes would often cost one.
 constexpr size_t kColSumBytes = 256;
-constexpr bool col_sum_separate(size_t base_bytes) { return base_bytes + kColSumBytes <= kLdsBytes; }
+constexpr bool col_sum_separate(size_t base_bytes) {
+  return base_bytes + kColSumBytes <= kLdsBytes &&
+         kLdsBytes / (base_bytes + kColSumBytes) == kLdsBytes / base_bytes;
+}
 
 }  // namespace sgpe

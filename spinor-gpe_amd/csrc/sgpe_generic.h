@@ -216,18 +216,26 @@ __global__ __launch_bounds__(kGenThreads) void gen_col_pass_kernel(const InstDev
   C* cur = kspace ? A : gen_fft<false>(A, B, f, W, 1, W, root);
   C* oth = cur == A ? B : A;
   const double* td = P.t_dense[comp];
-  const C* kxp = reinterpret_cast<const C*>(P.kx[d_prev][comp]);
-  const C* kyp = reinterpret_cast<const C*>(P.ky[d_prev][comp]);
-  const C* kxc = reinterpret_cast<const C*>(P.kx[d_cur][comp]);
-  const C* kyc = reinterpret_cast<const C*>(P.ky[d_cur][comp]);
+  const bool mid = mode != COL_EXIT;
+  const bool imag = P.imag != 0;
+  const bool want_s = mode == COL_MID_S;
+  // Kinetic factors as in col_kinetic: one of K_prev (closing pass), K_cur
+  // (state in k-space) and their product, except that imaginary time with S
+  // asked for applies the two in turn.
+  const bool both = imag && mid && want_s && !kspace;
+  const bool apply = mid || !kspace;
+  const bool one = !imag && (kspace || !mid);
+  const int d1 = kspace ? d_cur : d_prev;
+  const C* kx = reinterpret_cast<const C*>(one ? P.kx[d1][comp] : P.k2x[d_prev][d_cur][comp]);
+  const C* ky = reinterpret_cast<const C*>(one ? P.ky[d1][comp] : P.k2y[d_prev][d_cur][comp]);
   const R hp = (R)(0.5 * P.dt_sub[d_prev]);
   const R hc = (R)(0.5 * P.dt_sub[d_cur]);
-  const bool mid = mode == COL_MID;
+  const R h = (kspace ? (R)0 : hp) + (mid ? hc : (R)0);
   double v[2] = {0.0, 0.0};
   // Four elements per thread at a time: their table entries are read before
   // any of them is rewritten (see gen_copy_in); same order of operations.
   for (int e0 = threadIdx.x; e0 < cnt; e0 += 4 * (int)blockDim.x) {
-    C kp[4], kc[4];
+    C x[4], y[4];
     R tv[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -237,8 +245,8 @@ __global__ __launch_bounds__(kGenThreads) void gen_col_pass_kernel(const InstDev
       if (td) {
         tv[i] = (R)td[(size_t)jy * nx + jx];
       } else {
-        kp[i] = cmul(kxp[jx], kyp[jy]);
-        kc[i] = cmul(kxc[jx], kyc[jy]);
+        x[i] = kx[jx];
+        y[i] = ky[jy];
       }
     }
 #pragma unroll
@@ -246,27 +254,24 @@ __global__ __launch_bounds__(kGenThreads) void gen_col_pass_kernel(const InstDev
       const int e = e0 + i * (int)blockDim.x;
       if (e >= cnt) continue;
       C a = cur[e];
-      if (!kspace) {
-        C k;
-        if (td)
-          k = P.imag ? phase_op<R, true>(tv[i] * hp) : phase_op<R, false>(tv[i] * hp);
-        else
-          k = kp[i];
-        a = cmul(a, k);
+      if (imag) {
+        const R k1 = kspace ? (R)1 : td ? phase_op<R, true>(tv[i] * hp).x : x[i].x * y[i].x;
+        const R k2 = !mid ? (R)1 : td ? phase_op<R, true>(tv[i] * hc).x : x[i].y * y[i].y;
+        if (both || kspace) {
+          a = cscale(a, k1);
+          v[0] += norm2d<R>(a);
+          a = cscale(a, k2);
+        } else {
+          a = cscale(a, k1 * k2);
+        }
+      } else if (apply) {
+        a = cmul(a, td ? phase_op<R, false>(tv[i] * h) : cmul(x[i], y[i]));
       }
-      v[0] += norm2d<R>(a);
-      if (mid) {
-        C k;
-        if (td)
-          k = P.imag ? phase_op<R, true>(tv[i] * hc) : phase_op<R, false>(tv[i] * hc);
-        else
-          k = kc[i];
-        a = cmul(a, k);
-        v[1] += norm2d<R>(a);
-      }
+      v[1] += norm2d<R>(a);
       cur[e] = a;
     }
   }
+  if (!imag || !(both || kspace)) v[0] = v[1];
   __syncthreads();
   if (mid) cur = gen_fft<true>(cur, oth, f, W, 1, W, root);
   for (int e = threadIdx.x; e < cnt; e += blockDim.x) psi[(size_t)(e / W) * nx + (e % W)] = cur[e];

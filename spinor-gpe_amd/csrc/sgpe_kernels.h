@@ -272,43 +272,86 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 
 // Kinetic factors of the column pass on this thread's E points of column jx:
 // the closing K of the previous sub-step (unless the state is already in
-// k-space) with the S sum after it, then the opening K of this sub-step with
-// the NRM sum after it (mid). DENSE: K from the dense T array, else from the
-// separable tables. The two block-uniform choices (kspace, mid) are taken
-// once, around whole point loops: tested per point, they put every table
-// read in a block of its own with its own wait, a chain of 2E dependent LDS
-// round trips (≈1 µs of a 512-point column pass). The sums run over the
-// points in the same order either way. DENSE reads T in each loop (the second
-// read hits the cache) rather than keeping E values live across both.
-// KYG: the y tables are in global memory (else staged in LDS).
+// k-space: `kspace`) and the opening K of this one (`mid`), with the norm sums.
+// S is the norm between the two, NRM the one after both; want_s: S is asked
+// for (populations, once a full step).
+//  - Real time: |K| = 1, so S = NRM, and both half steps are one phase from one
+//    pair of tables (k2x, k2y): 10 instructions a point where the two factors
+//    and two sums took 22.
+//  - Imaginary time: both K are real; the tables hold them as the parts of one
+//    entry, and without S their product is applied at once (8 instructions).
+// DENSE: K from the dense T array. kx, ky: the table values of this column and
+// the y table (KYG: in global memory, else staged in LDS); in real time with
+// the state in k-space they are those of K_cur alone.
+// The uniform choices are taken around whole point loops: tested per point,
+// they put every table read in a block of its own with its own wait, a chain
+// of dependent LDS round trips.
 template <typename R, int E, int T, bool DENSE, bool IMAG, bool KYG, typename C>
 __device__ __forceinline__ void col_kinetic(C (&a)[E], int t, int nx, int jx, const double* __restrict__ td, R hp,
-                                            R hc, C kxp, C kxc, const C* kyp, const C* kyc, bool kspace, bool mid,
+                                            R hc, C kx, const C* ky, bool kspace, bool mid, bool want_s,
                                             double& s_acc, double& n_acc) {
-  if (!kspace) {
+  auto yval = [&](int j) -> C { return KYG ? ld_global(ky + t + j * T) : ky[t + j * T]; };
+  auto dense = [&](int j, R h) -> C {
+    return phase_op<R, IMAG>((R)ld_global(td + (size_t)(t + j * T) * nx + jx) * h);
+  };
+  if (kspace && !mid) {
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      C k;
-      if constexpr (DENSE)
-        k = phase_op<R, IMAG>((R)ld_global(td + (size_t)(t + j * T) * nx + jx) * hp);
-      else
-        k = cmul(kxp, KYG ? ld_global(kyp + t + j * T) : kyp[t + j * T]);
-      a[j] = cmul(a[j], k);
-    }
+    for (int j = 0; j < E; ++j) n_acc += norm2d<R>(a[j]);
+    s_acc = n_acc;
+    return;
   }
-#pragma unroll
-  for (int j = 0; j < E; ++j) s_acc += norm2d<R>(a[j]);
-  if (mid) {
+  if constexpr (!IMAG) {
+    const R h = (kspace ? (R)0 : hp) + (mid ? hc : (R)0);
 #pragma unroll
     for (int j = 0; j < E; ++j) {
       C k;
       if constexpr (DENSE)
-        k = phase_op<R, IMAG>((R)ld_global(td + (size_t)(t + j * T) * nx + jx) * hc);
+        k = dense(j, h);
       else
-        k = cmul(kxc, KYG ? ld_global(kyc + t + j * T) : kyc[t + j * T]);
+        k = cmul(kx, yval(j));
       a[j] = cmul(a[j], k);
       n_acc += norm2d<R>(a[j]);
     }
+    s_acc = n_acc;
+  } else if (mid && want_s && !kspace) {
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      R k1, k2;
+      if constexpr (DENSE) {
+        k1 = dense(j, hp).x;
+        k2 = dense(j, hc).x;
+      } else {
+        const C y = yval(j);
+        k1 = kx.x * y.x;
+        k2 = kx.y * y.y;
+      }
+      a[j] = cscale(a[j], k1);
+      s_acc += norm2d<R>(a[j]);
+      a[j] = cscale(a[j], k2);
+      n_acc += norm2d<R>(a[j]);
+    }
+  } else {
+    if (kspace) {
+#pragma unroll
+      for (int j = 0; j < E; ++j) s_acc += norm2d<R>(a[j]);
+    }
+    const R h = (kspace ? (R)0 : hp) + (mid ? hc : (R)0);
+    // One factor a point: K_prev K_cur, or one of them with 1 for the other.
+    const R x1 = kspace ? (R)1 : kx.x, x2 = mid ? kx.y : (R)1;
+    const R x12 = x1 * x2;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      R k;
+      if constexpr (DENSE) {
+        k = dense(j, h).x;
+      } else {
+        const C y = yval(j);
+        k = x12 * ((kspace ? (R)1 : y.x) * (mid ? y.y : (R)1));
+      }
+      a[j] = cscale(a[j], k);
+      n_acc += norm2d<R>(a[j]);
+    }
+    if (!kspace) s_acc = n_acc;
   }
 }
 
@@ -325,14 +368,14 @@ __device__ __forceinline__ void col_item(const InstDev& P, typename Cx<R>::T* __
   typedef typename Cx<R>::T C;
   typedef LdsView<W, 1 << 30, 0> V;
   constexpr int T = N / E;
-  // LDS: [W*N exchange][N twiddles][N ky_prev][N ky_cur][sums] (tables and
-  // a separate sum slot when they fit). GKY: the two y phase tables stay in
-  // global memory (cache resident) even where they would fit, which leaves
-  // LDS for more workgroups per CU in batched plans.
+  // LDS: [W*N exchange][N twiddles][N y phase table][sums] (tables and a
+  // separate sum slot when they fit). GKY: the y phase table stays in global
+  // memory (cache resident) even where it would fit, which leaves LDS for more
+  // workgroups per CU in batched plans.
   constexpr size_t kData = (size_t)W * N * sizeof(C);
   constexpr bool kTw = tw_in_lds(kData, N, sizeof(C));
-  constexpr bool kKy = !GKY && kTw && kData + 3 * (size_t)N * sizeof(C) <= kLdsBytes;
-  constexpr size_t kBase = kData + (kTw ? (size_t)N * sizeof(C) : 0) + (kKy ? 2 * (size_t)N * sizeof(C) : 0);
+  constexpr bool kKy = !GKY && kTw && kData + 2 * (size_t)N * sizeof(C) <= kLdsBytes;
+  constexpr size_t kBase = kData + (kTw ? (size_t)N * sizeof(C) : 0) + (kKy ? (size_t)N * sizeof(C) : 0);
   constexpr bool kSumSep = col_sum_separate(kBase);
   // The W*T threads of a tile interleave its W columns, so a column's
   // transform lies within one wave when the whole tile does.
@@ -363,24 +406,23 @@ __device__ __forceinline__ void col_item(const InstDev& P, typename Cx<R>::T* __
     for (int j = 0; j < E; ++j) a[j] = ld_global(col + (size_t)(t + j * T) * nx);
   }
   const double* td = P.t_dense[comp];
-  C kxp = C{(R)1, (R)0}, kxc = C{(R)1, (R)0};
-  TableStage<kKy, N, kBlock, C> sp, sc_;
+  const bool mid = mode != COL_EXIT;
+  const bool imag = P.imag != 0;
+  C kx = C{(R)1, (R)0};
+  TableStage<kKy, N, kBlock, C> sky;
   TableStage<kTw, N, kBlock, C> stw;
-  if (!td) {
-    kxp = ld_global(reinterpret_cast<const C*>(P.kx[d_prev][comp]) + jx);
-    kxc = ld_global(reinterpret_cast<const C*>(P.kx[d_cur][comp]) + jx);
-  }
-  // The y-tables are staged unconditionally (a conditional fill puts the
-  // staging registers in scratch); without them (dense kinetic operator) the
-  // twiddle table, also N entries, stands in and the copies go unused.
-  sp.load(td ? tws : reinterpret_cast<const C*>(P.ky[d_prev][comp]));
-  sc_.load(td ? tws : reinterpret_cast<const C*>(P.ky[d_cur][comp]));
+  // Both half steps' tables; the closing pass in real time takes K_prev's.
+  const bool one = !mid && !imag;
+  if (!td) kx = ld_global(reinterpret_cast<const C*>(one ? P.kx[d_prev][comp] : P.k2x[d_prev][d_cur][comp]) + jx);
+  // The y table is staged unconditionally (a conditional fill puts the
+  // staging registers in scratch); without it (dense kinetic operator) the
+  // twiddle table, also N entries, stands in and the copy goes unused.
+  sky.load(td ? tws : reinterpret_cast<const C*>(one ? P.ky[d_prev][comp] : P.k2y[d_prev][d_cur][comp]));
   stw.load(tws);
   const int gk = gate();
   if (gk < 0) return;
   const bool kspace = gk != 0;
-  const C* kyp = sp.store(sm + W * N + N);
-  const C* kyc = sc_.store(sm + W * N + 2 * N);
+  const C* ky = sky.store(sm + W * N + N);
   const C* tw = stw.store(sm + W * N);
 
   if (!kspace) {
@@ -393,24 +435,33 @@ __device__ __forceinline__ void col_item(const InstDev& P, typename Cx<R>::T* __
   double s_acc = 0.0, n_acc = 0.0;
   const R hp = (R)(0.5 * P.dt_sub[d_prev]);
   const R hc = (R)(0.5 * P.dt_sub[d_cur]);
-  const bool mid = mode == COL_MID;
-  if (!DENSE || !td)
-    col_kinetic<R, E, T, false, false, !kKy>(a, t, nx, jx, nullptr, hp, hc, kxp, kxc, kyp, kyc, kspace, mid, s_acc,
-                                           n_acc);
-  else if constexpr (DENSE) {
-    if (P.imag)
-      col_kinetic<R, E, T, true, true, !kKy>(a, t, nx, jx, td, hp, hc, kxp, kxc, kyp, kyc, kspace, mid, s_acc, n_acc);
+  const bool want_s = mode == COL_MID_S;
+  if (!DENSE || !td) {
+    if (imag) {
+      col_kinetic<R, E, T, false, true, !kKy>(a, t, nx, jx, nullptr, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
+    } else if (kspace) {  // first pass from k-space: K_cur's own tables
+      const C kc = ld_global(reinterpret_cast<const C*>(P.kx[d_cur][comp]) + jx);
+      col_kinetic<R, E, T, false, false, true>(a, t, nx, jx, nullptr, hp, hc, kc,
+                                               reinterpret_cast<const C*>(P.ky[d_cur][comp]), true, mid, want_s,
+                                               s_acc, n_acc);
+    } else {
+      col_kinetic<R, E, T, false, false, !kKy>(a, t, nx, jx, nullptr, hp, hc, kx, ky, false, mid, want_s, s_acc,
+                                               n_acc);
+    }
+  } else if constexpr (DENSE) {
+    if (imag)
+      col_kinetic<R, E, T, true, true, !kKy>(a, t, nx, jx, td, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
     else
-      col_kinetic<R, E, T, true, false, !kKy>(a, t, nx, jx, td, hp, hc, kxp, kxc, kyp, kyc, kspace, mid, s_acc,
-                                              n_acc);
+      col_kinetic<R, E, T, true, false, !kKy>(a, t, nx, jx, td, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
   }
-  // Columns of 1024 points and more: an opaque copy of t for the inverse
-  // transform and the stores, so their addresses are recomputed rather than
-  // held since the loads (as in row_item; 2-5 % per pass there, while
-  // shorter batched columns lose 1-2 % to the recomputation).
+  // Columns of 1024 points and more, and complex64 columns: an opaque copy of
+  // t for the inverse transform and the stores, so their addresses are
+  // recomputed rather than held since the loads (as in row_item; 2-5 % per
+  // pass at 1024 points and more; complex64 512-point columns 82 -> 60
+  // registers, 8 waves per SIMD instead of 5).
   int tf = t;
-  if constexpr (N >= 1024) asm volatile("" : "+v"(tf));
-  if (mode == COL_MID) fft_run<N, E, true, V, kWave>(a, tf, tw, lds);
+  if constexpr (N >= 1024 || sizeof(C) == 8) asm volatile("" : "+v"(tf));
+  if (mid) fft_run<N, E, true, V, kWave>(a, tf, tw, lds);
   if constexpr ((CM & CM_STORE) != 0) {
 #pragma unroll
     for (int j = 0; j < E; ++j) cb.store<C>(cbase + (uint32_t)((tf + j * T) * nx * sizeof(C)), a[j]);
@@ -422,11 +473,23 @@ __device__ __forceinline__ void col_item(const InstDev& P, typename Cx<R>::T* __
     for (int j = 0; j < E; ++j) st_global(col + (size_t)(tf + j * T) * nx, a[j]);
   }
 
+  // S differs from NRM only in imaginary time with both factors present; one
+  // sum otherwise.
   double v[2] = {s_acc, n_acc};
-  if constexpr (kSumSep)
-    block_sum_thread0<2>(v, reinterpret_cast<double*>(reinterpret_cast<char*>(smem) + kBase));
-  else
-    block_sum<2>(v, smem);
+  double* const sums = kSumSep ? reinterpret_cast<double*>(reinterpret_cast<char*>(smem) + kBase) : smem;
+  if (imag && mid && (want_s || kspace)) {
+    if constexpr (kSumSep)
+      block_sum_thread0<2>(v, sums);
+    else
+      block_sum<2>(v, sums);
+  } else {
+    double w[1] = {n_acc};
+    if constexpr (kSumSep)
+      block_sum_thread0<1>(w, sums);
+    else
+      block_sum<1>(w, sums);
+    v[0] = v[1] = w[0];
+  }
   if (threadIdx.x == 0) {
     const int nt = nx / W;
     double* ps = P.part + PART_S * 2 * nt + comp * nt + tile;

@@ -179,7 +179,7 @@ __global__ __launch_bounds__(RROWS*(N / RE)) void persist_steps_kernel(PersistAr
         C* psi = reinterpret_cast<C*>(a.direct_psi ? a.direct_psi : P.psi);
         const int kspace = sub == 0 ? s_kspace[li] : 0;
         const int comp = r / kTiles;
-        col_item<R, N, CE, CW, false, CM>(P, psi, N, twy, COL_MID, dprev, dur, a.col_stream, comp,
+        col_item<R, N, CE, CW, false, CM>(P, psi, N, twy, j == 0 ? COL_MID_S : COL_MID, dprev, dur, a.col_stream, comp,
                                       xcd_tile(r - comp * kTiles, kTiles), smem, [&]() -> int { return kspace; });
         persist_signal(&a.sync[inst].col_done);
       }
