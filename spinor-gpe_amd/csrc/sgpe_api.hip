@@ -16,6 +16,7 @@
 
 #include "../../include/sgpe.h"
 #include "sgpe_generic.h"
+#include "sgpe_mixed.h"
 #include "sgpe_persist.h"
 #include "sgpe_registry.h"
 
@@ -187,6 +188,104 @@ static int gen_col_width(int n, int nx, size_t cs) {
   return 1;
 }
 
+// ---- mixed-radix register kernels (sgpe_mixed.h)
+
+// Splits m into ns radices of 2 .. kMixMaxRadix (non-increasing, at most
+// `top`) of the smallest sum; false if there is none.
+static bool mix_split(int m, int ns, int top, int* out, int* sum) {
+  if (ns == 0) {
+    *sum = 0;
+    return m == 1;
+  }
+  bool found = false;
+  for (int r = std::min(top, m); r >= 2; --r) {
+    int rest[kMixMaxStages], s = 0;
+    if (m % r || !mix_split(m / r, ns - 1, r, rest, &s) || (found && s + r >= *sum)) continue;
+    found = true;
+    *sum = s + r;
+    out[0] = r;
+    for (int i = 1; i < ns; ++i) out[i] = rest[i - 1];
+  }
+  return found;
+}
+
+static unsigned mix_magic(int d) { return (unsigned)((1ull << 32) / (unsigned)d + 1); }
+
+// Radices of an n-point transform: the fewest stages, then the smallest sum of
+// radices, then the smallest last radix from 4 on (of at most kMixMidRadix):
+// the last stage does both transforms' butterflies and the pointwise block, so
+// many items of few points there keep more threads busy. Stage 0, whose outputs go to LDS a
+// radix apart, takes the radix with the fewest factors of two (bank
+// conflicts). ns = 0: not a length of these kernels.
+static MixFft mix_factor(int n) {
+  MixFft f;
+  std::memset(&f, 0, sizeof(f));
+  if (n < kMixMinLen || n > kMixMaxLen) return f;
+  for (int ns = 2; ns <= kMixMaxStages && !f.ns; ++ns) {
+    int best = 0, r[kMixMaxStages];
+    for (int i = 2; i <= kMixMidRadix; ++i) {
+      const int last = i <= kMixMidRadix - 2 ? i + 2 : kMixMidRadix + 2 - i;  // 4, 5, ... kMixMidRadix, 3, 2
+      int t[kMixMaxStages], sum = 0;
+      if (n % last || !mix_split(n / last, ns - 1, kMixMaxRadix, t, &sum)) continue;
+      if (best && sum + last >= best) continue;
+      best = sum + last;
+      for (int i = 0; i < ns - 1; ++i) r[i] = t[i];
+      r[ns - 1] = last;
+    }
+    if (!best) continue;
+    for (int i = 1; i < ns - 1; ++i)
+      if ((r[i] & -r[i]) < (r[0] & -r[0])) std::swap(r[0], r[i]);
+    f.n = n;
+    f.ns = ns;
+    for (int i = 0, span = 1; i < ns; span *= r[i++]) {
+      f.st[i].radix = r[i];
+      f.st[i].span = span;
+      f.st[i].nb = n / r[i];
+      f.st[i].off = span - 1;
+      f.st[i].div_span = mix_magic(span);
+      f.st[i].div_nb = mix_magic(n / r[i]);
+    }
+  }
+  return f;
+}
+
+// LDS of `batch` transforms: data, twiddles, sums.
+static size_t mix_lds(int batch, int n, size_t cs) { return (size_t)(batch + 1) * n * cs + 256; }
+
+// Whether `batch` transforms fit a workgroup: LDS, and an inner stage's
+// butterflies within kMixThreads threads (one each).
+static bool mix_fits(const MixFft& f, int batch, size_t cs, size_t lds_max) {
+  if (mix_lds(batch, f.n, cs) > lds_max) return false;
+  for (int s = 1; s < f.ns - 1; ++s)
+    if (f.st[s].nb * batch > kMixThreads) return false;
+  return true;
+}
+
+// Threads of a workgroup of `batch` transforms (`mid` of them in the last
+// stage: rows take two components together): all inner butterflies at once,
+// the outer stages in as few even rounds.
+static int mix_threads(const MixFft& f, int batch, int mid) {
+  int t = 64;
+  for (int s = 1; s < f.ns - 1; ++s) t = std::max(t, f.st[s].nb * batch);
+  const int outer = std::max(f.st[0].nb * batch, f.st[f.ns - 1].nb * mid);
+  const int rounds = (outer + kMixThreads - 1) / kMixThreads;
+  t = std::max(t, (outer + rounds - 1) / rounds);
+  return std::min((t + 63) / 64 * 64, kMixThreads);
+}
+
+// Transforms per workgroup out of `count` (a divisor of it), the widest that
+// still makes `want` workgroups of `copies` x count / batch, at most `most`;
+// at least `least` (coalescing) where LDS allows that. 0: none fits.
+static int mix_batch(const MixFft& f, int count, long copies, size_t cs, int least, int most, int per, long want) {
+  const size_t lds_max = 80 * 1024;
+  int best = 0;
+  for (int b = 1; b <= most; ++b) {
+    if (count % b || !mix_fits(f, b * per, cs, b == 1 ? kLdsBytes : lds_max)) continue;
+    if (!best || b <= least || copies * (count / b) >= want) best = b;
+  }
+  return best;
+}
+
 // A compiled shape of pass `kind` for length n whose tile divides `other`:
 // the given default if it does, else the entry with the same radix and the
 // widest tile that does, else any radix. False: none.
@@ -310,45 +409,50 @@ static int ctx_twiddles(sgpe_ctx* ctx, int prec, int n, int e, const void** out)
   return SGPE_OK;
 }
 
-// Roots of unity root[m] = exp(-2 pi i m / n), m < n, of the runtime-length
-// kernels (any even n): angles reduced exactly to [0, pi/4] (4m mod n and
-// its complement are integers), long double cos/sin there, then the
-// quarter-turn rotation; quarter turns come out exact.
-static int ctx_roots(sgpe_ctx* ctx, int prec, int n, const void** out) {
-  const int key = (prec * 8192 + n) * 32;  // e = 0: no compiled shape uses it
+// exp(-2 pi i m / n): the angle reduced exactly to [0, pi/4] (4m mod n and its
+// complement are integers), long double cos/sin there, then the quarter-turn
+// rotation; quarter turns come out exact.
+static void root_of_unity(int m, int n, double* re, double* im) {
+  const long double half_pi = 1.5707963267948966192313216916397514L;
+  const long long u = 4LL * (m % n);  // angle = (pi / 2) u / n
+  const int quad = (int)(u / n);      // whole quarter turns
+  const long long rem = u - (long long)quad * n;
+  long double c, sn;                  // cos, sin of (pi / 2) rem / n
+  if (2 * rem <= n) {
+    const long double a = half_pi * (long double)rem / (long double)n;
+    c = cosl(a);
+    sn = sinl(a);
+  } else {
+    const long double a = half_pi * (long double)(n - rem) / (long double)n;
+    c = sinl(a);
+    sn = cosl(a);
+  }
+  for (int r = 0; r < quad; ++r) {  // rotate by pi / 2: (c, s) -> (-s, c)
+    const long double t = c;
+    c = -sn;
+    sn = t;
+  }
+  *re = (double)c;
+  *im = (double)-sn;  // exp(-i angle)
+}
+
+// Device table of n complex entries value(i, &re, &im), cached under `key`.
+template <class F> static int ctx_table(sgpe_ctx* ctx, int key, int prec, int n, F value, const void** out) {
   auto it = ctx->tw.find(key);
   if (it != ctx->tw.end()) {
     *out = it->second;
     return SGPE_OK;
   }
   std::vector<char> host(n * csize(prec));
-  const long double half_pi = 1.5707963267948966192313216916397514L;
-  for (int m = 0; m < n; ++m) {
-    const long long u = 4LL * m;      // angle = (pi / 2) u / n
-    const int quad = (int)(u / n);    // whole quarter turns
-    const long long rem = u - (long long)quad * n;
-    long double c, sn;                // cos, sin of (pi / 2) rem / n
-    if (2 * rem <= n) {
-      const long double a = half_pi * (long double)rem / (long double)n;
-      c = cosl(a);
-      sn = sinl(a);
-    } else {
-      const long double a = half_pi * (long double)(n - rem) / (long double)n;
-      c = sinl(a);
-      sn = cosl(a);
-    }
-    for (int r = 0; r < quad; ++r) {  // rotate by pi / 2: (c, s) -> (-s, c)
-      const long double t = c;
-      c = -sn;
-      sn = t;
-    }
-    const double re = (double)c, im = (double)-sn;  // exp(-i angle)
+  for (int i = 0; i < n; ++i) {
+    double re, im;
+    value(i, &re, &im);
     if (prec == SGPE_C128) {
-      ((double*)host.data())[2 * m] = re;
-      ((double*)host.data())[2 * m + 1] = im;
+      ((double*)host.data())[2 * i] = re;
+      ((double*)host.data())[2 * i + 1] = im;
     } else {
-      ((float*)host.data())[2 * m] = (float)re;
-      ((float*)host.data())[2 * m + 1] = (float)im;
+      ((float*)host.data())[2 * i] = (float)re;
+      ((float*)host.data())[2 * i + 1] = (float)im;
     }
   }
   void* d = nullptr;
@@ -358,6 +462,29 @@ static int ctx_roots(sgpe_ctx* ctx, int prec, int n, const void** out) {
   ctx->tw[key] = d;
   *out = d;
   return SGPE_OK;
+}
+
+// Roots of unity root[m] = exp(-2 pi i m / n), m < n, of the runtime-length
+// kernels (any even n).
+static int ctx_roots(sgpe_ctx* ctx, int prec, int n, const void** out) {
+  const int key = (prec * 8192 + n) * 32;  // e = 0: no compiled shape uses it
+  return ctx_table(ctx, key, prec, n, [n](int m, double* re, double* im) { root_of_unity(m, n, re, im); }, out);
+}
+
+// Stage-major twiddles of the mixed-radix kernels: the stage of span L and
+// radix R keeps w_{L R}^{r k} (k < L, 1 <= r < R) at (L - 1) + k (R - 1) +
+// (r - 1).
+static int ctx_mix_twiddles(sgpe_ctx* ctx, int prec, const MixFft& f, const void** out) {
+  const int n = f.n;
+  const int key = (prec * 8192 + n) * 32 + 17;  // compiled shapes: e <= 16
+  std::vector<int> power(n, 0);  // entry i is exp(-2 pi i power[i] / n)
+  for (int s = 0; s < f.ns; ++s) {
+    const int L = f.st[s].span, R = f.st[s].radix;
+    for (int k = 0; k < L; ++k)
+      for (int r = 1; r < R; ++r) power[f.st[s].off + k * (R - 1) + r - 1] = r * k * (n / (L * R));
+  }
+  return ctx_table(ctx, key, prec, n,
+                   [&](int i, double* re, double* im) { root_of_unity(power[i], n, re, im); }, out);
 }
 
 // Dynamic LDS of a kernel with data_bytes of exchange buffers for n-point
@@ -436,6 +563,10 @@ struct sgpe_plan {
   // with -W columns per block; col_w keeps the positive tile width).
   bool col_gky = false;
   GenFft gfx{}, gfy{};
+  // The mixed-radix kernels stand in for the runtime-length ones where the
+  // length allows (ns > 0); mix_rows: rows per workgroup.
+  MixFft mfx{}, mfy{};
+  int mix_rows = 1;
   const void* root_x = nullptr;
   const void* root_y = nullptr;
   InstDev* d_inst = nullptr;
@@ -479,8 +610,24 @@ static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col
   if ((gx && !gen_length_ok(p->nx)) || (gy && !gen_length_ok(p->ny)))
     return fail(SGPE_E_UNSUPPORTED, "no compiled FFT tile of this length divides the other grid axis");
   const size_t cs = csize(p->prec);
-  if (gx) row_rows = 1;
-  if (gy) col_w = gen_col_width(p->ny, p->nx, cs);
+  // Without compiled passes: mixed-radix kernels where the length splits, else
+  // the runtime-length ones. Tiles as wide as leaves two workgroups per CU;
+  // columns at least 64 bytes.
+  MixFft mx{}, my{};
+  int mrows = 0, mw = 0;
+  if (gx) {
+    mx = mix_factor(p->nx);
+    if (mx.ns) mrows = mix_batch(mx, p->ny, p->nslots, cs, 1, 4, 2, 2L * std::max(p->ctx->n_cu, 1));
+    if (!mrows) mx.ns = 0;
+    row_rows = 1;
+  }
+  if (gy) {
+    my = mix_factor(p->ny);
+    if (my.ns)
+      mw = mix_batch(my, p->nx, 2L * p->nslots, cs, (int)(64 / cs), (int)(128 / cs), 1, 2L * std::max(p->ctx->n_cu, 1));
+    if (!mw) my.ns = 0;
+    col_w = my.ns ? mw : gen_col_width(p->ny, p->nx, cs);
+  }
   const KEntry* r = gx ? nullptr : find_entry(K_ROW, p->prec, p->nx, row_e, row_rows);
   const KEntry* c = gy ? nullptr : find_entry(K_COL, p->prec, p->ny, col_e, col_w);
   if ((!gx && !r) || (!gy && !c)) return fail(SGPE_E_UNSUPPORTED, "FFT shape not compiled for this grid/precision");
@@ -490,12 +637,20 @@ static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col
   const size_t row_data = (size_t)std::abs(row_rows) * 2 * p->nx * cs;
   const size_t col_data = (size_t)col_w * p->ny * cs;
   if (row_data > kMaxLds || col_data > kMaxLds) return fail(SGPE_E_UNSUPPORTED, "FFT shape exceeds LDS");
-  const size_t rl = gx ? gen_rows_lds(2, p->nx, cs) : row_pass_lds(row_e, row_rows, p->nx, cs);
-  const size_t cl = gy ? gen_cols_lds(col_w, p->ny, cs) : col_lds_bytes(col_w, p->ny, cs, gky);
+  const size_t rl = mx.ns ? mix_lds(2 * mrows, p->nx, cs)
+                    : gx ? gen_rows_lds(2, p->nx, cs) : row_pass_lds(row_e, row_rows, p->nx, cs);
+  const size_t cl = my.ns ? mix_lds(mw, p->ny, cs)
+                    : gy ? gen_cols_lds(col_w, p->ny, cs) : col_lds_bytes(col_w, p->ny, cs, gky);
   if (rl > kMaxLds || cl > kMaxLds) return fail(SGPE_E_UNSUPPORTED, "FFT shape exceeds LDS");
   int rc = SGPE_OK;
   const void *twx = nullptr, *twy = nullptr;
-  if (gx) {
+  const bool f64 = p->prec == SGPE_C128;
+  auto mix_kernel = [f64](int which) { return f64 ? MixKernels<double>::kernel(which) : MixKernels<float>::kernel(which); };
+  if (mx.ns) {
+    rc = set_lds_attr(mix_kernel(MIX_ROW), rl);
+    if (!rc) rc = set_lds_attr(mix_kernel(MIX_ROW_GENERAL), rl);
+    if (!rc) rc = ctx_mix_twiddles(p->ctx, p->prec, mx, &twx);
+  } else if (gx) {
     rc = set_lds_attr(p->prec == SGPE_C128 ? (const void*)gen_row_pass_kernel<double>
                                            : (const void*)gen_row_pass_kernel<float>, rl);
     if (!rc) rc = ctx_roots(p->ctx, p->prec, p->nx, &twx);
@@ -505,7 +660,10 @@ static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col
     if (!rc) rc = ctx_twiddles(p->ctx, p->prec, p->nx, row_e, &twx);
   }
   if (rc) return rc;
-  if (gy) {
+  if (my.ns) {
+    rc = set_lds_attr(mix_kernel(MIX_COL), cl);
+    if (!rc) rc = ctx_mix_twiddles(p->ctx, p->prec, my, &twy);
+  } else if (gy) {
     rc = set_lds_attr(p->prec == SGPE_C128 ? (const void*)gen_col_pass_kernel<double>
                                            : (const void*)gen_col_pass_kernel<float>, cl);
     if (!rc) rc = ctx_roots(p->ctx, p->prec, p->ny, &twy);
@@ -519,6 +677,9 @@ static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col
   p->gen_y = gy;
   p->gfx = gen_factor(p->nx);
   p->gfy = gen_factor(p->ny);
+  p->mfx = mx;
+  p->mfy = my;
+  p->mix_rows = mrows;
   p->tw_x = gx ? nullptr : twx;
   p->tw_y = gy ? nullptr : twy;
   p->root_x = gx ? twx : nullptr;
@@ -574,6 +735,13 @@ static void* direct_state(const sgpe_plan* p) {
 
 static void launch_col(sgpe_plan* p, hipStream_t s, int mode, int dprev, int dcur, hipEvent_t e0 = nullptr,
                        hipEvent_t e1 = nullptr) {
+  if (p->mfy.ns) {
+    const auto launch = p->prec == SGPE_C128 ? MixKernels<double>::col : MixKernels<float>::col;
+    launch(dim3(p->nx / p->col_w, 2, p->nlaunch), dim3(mix_threads(p->mfy, p->col_w, p->col_w)),
+           mix_lds(p->col_w, p->ny, csize(p->prec)), s, e0, e1, p->d_inst, p->d_run, p->mfy, p->root_y, p->col_w,
+           mix_magic(p->col_w), mode, dprev, dcur);
+    return;
+  }
   if (p->gen_y) {
     const size_t lds = gen_cols_lds(p->col_w, p->ny, csize(p->prec));
     const dim3 grid(p->nx / p->col_w, 2, p->nlaunch), block(kGenThreads);
@@ -594,6 +762,13 @@ static void launch_col(sgpe_plan* p, hipStream_t s, int mode, int dprev, int dcu
 
 static void launch_row(sgpe_plan* p, hipStream_t s, int dur, int first, hipEvent_t e0 = nullptr,
                        hipEvent_t e1 = nullptr) {
+  if (p->mfx.ns) {
+    const auto launch = p->prec == SGPE_C128 ? MixKernels<double>::row : MixKernels<float>::row;
+    launch(dim3(p->ny / p->mix_rows, 1, p->nlaunch), dim3(mix_threads(p->mfx, 2 * p->mix_rows, p->mix_rows)),
+           mix_lds(2 * p->mix_rows, p->nx, csize(p->prec)), s, e0, e1, p->d_inst, p->d_run, p->mfx, p->root_x,
+           p->mix_rows, dur, first, p->col_w, p->general_row);
+    return;
+  }
   if (p->gen_x) {
     const size_t lds = gen_rows_lds(2, p->nx, csize(p->prec));
     const dim3 grid(p->ny, 1, p->nlaunch), block(kGenThreads);
@@ -1159,24 +1334,50 @@ int sgpe_fft2(sgpe_ctx* ctx, int precision, int ny, int nx, int n_arrays, void* 
     if ((gx && !gen_length_ok(nx)) || (gy && !gen_length_ok(ny)))
       return fail(SGPE_E_UNSUPPORTED, "no compiled FFT tile of this length divides the other grid axis");
     if (gy) cw = gen_col_width(ny, nx, cs);
+    MixFft mx{}, my{};  // mixed-radix kernels where the length splits
+    int mrows = 0, mw = 0;
+    const long per_launch = std::min(n_arrays, 2), want = 2L * std::max(ctx->n_cu, 1);
+    if (gx) {
+      mx = mix_factor(nx);
+      if (mx.ns) mrows = mix_batch(mx, ny, per_launch, cs, 1, 8, 1, want);
+      if (!mrows) mx.ns = 0;
+    }
+    if (gy) {
+      my = mix_factor(ny);
+      if (my.ns) mw = mix_batch(my, nx, per_launch, cs, (int)(64 / cs), (int)(128 / cs), 1, want);
+      if (!mw) my.ns = 0;
+    }
     const KEntry* fr = gx ? nullptr : find_entry(K_FROW, precision, nx, re, rr);
     const KEntry* fc = gy ? nullptr : find_entry(K_FCOL, precision, ny, ce, cw);
-    const size_t rl = gx ? gen_rows_lds(1, nx, cs) : lds_bytes((size_t)rr * nx * cs, nx, cs);
-    const size_t cl = gy ? gen_cols_lds(cw, ny, cs) : lds_bytes((size_t)cw * ny * cs, ny, cs);
-    const void* grk = f64 ? (const void*)gen_fft_rows_kernel<double> : (const void*)gen_fft_rows_kernel<float>;
-    const void* gck = f64 ? (const void*)gen_fft_cols_kernel<double> : (const void*)gen_fft_cols_kernel<float>;
+    const size_t rl = mx.ns ? mix_lds(mrows, nx, cs)
+                      : gx ? gen_rows_lds(1, nx, cs) : lds_bytes((size_t)rr * nx * cs, nx, cs);
+    const size_t cl = my.ns ? mix_lds(mw, ny, cs)
+                      : gy ? gen_cols_lds(cw, ny, cs) : lds_bytes((size_t)cw * ny * cs, ny, cs);
+    auto mix_kernel = [f64](int which) { return f64 ? MixKernels<double>::kernel(which) : MixKernels<float>::kernel(which); };
+    const void* grk = mx.ns ? mix_kernel(inverse ? MIX_FFT_ROWS_INV : MIX_FFT_ROWS)
+                      : f64 ? (const void*)gen_fft_rows_kernel<double> : (const void*)gen_fft_rows_kernel<float>;
+    const void* gck = my.ns ? mix_kernel(inverse ? MIX_FFT_COLS_INV : MIX_FFT_COLS)
+                      : f64 ? (const void*)gen_fft_cols_kernel<double> : (const void*)gen_fft_cols_kernel<float>;
     int rc = set_lds_attr(gx ? grk : fr->kernel, rl);
     if (rc) return rc;
     if ((rc = set_lds_attr(gy ? gck : fc->kernel, cl))) return rc;
     const void *twx, *twy;
-    if ((rc = gx ? ctx_roots(ctx, precision, nx, &twx) : ctx_twiddles(ctx, precision, nx, re, &twx))) return rc;
-    if ((rc = gy ? ctx_roots(ctx, precision, ny, &twy) : ctx_twiddles(ctx, precision, ny, ce, &twy))) return rc;
+    rc = mx.ns ? ctx_mix_twiddles(ctx, precision, mx, &twx)
+         : gx ? ctx_roots(ctx, precision, nx, &twx) : ctx_twiddles(ctx, precision, nx, re, &twx);
+    if (rc) return rc;
+    rc = my.ns ? ctx_mix_twiddles(ctx, precision, my, &twy)
+         : gy ? ctx_roots(ctx, precision, ny, &twy) : ctx_twiddles(ctx, precision, ny, ce, &twy);
+    if (rc) return rc;
     const GenFft gfx = gen_factor(nx), gfy = gen_factor(ny);
     const double c = dx * dy / (2.0 * M_PI);
     hipStream_t st = ctx->stream;
     // k arrays (1 or 2) of the pair io per launch, array blockIdx.z.
+    const auto mix_fft = f64 ? MixKernels<double>::fft : MixKernels<float>::fft;
     auto rows = [&](const FftPair& io, int k, int inv, double scale) {
-      if (!gx) {
+      if (mx.ns) {
+        mix_fft(dim3(ny / mrows, 1, k), dim3(mix_threads(mx, mrows, mrows)), rl, st, io, mx, twx, nx, mrows,
+                mix_magic(mrows), true, inv != 0, scale);
+      } else if (!gx) {
         ((FRowFn)fr->launch)(dim3(ny / rr, 1, k), dim3(rr * (nx / re)), rl, st, io, inv, 1, scale, twx);
       } else if (f64) {
         hipLaunchKernelGGL(gen_fft_rows_kernel<double>, dim3(ny, 1, k), dim3(kGenThreads), rl, st, io, gfx,
@@ -1187,7 +1388,10 @@ int sgpe_fft2(sgpe_ctx* ctx, int precision, int ny, int nx, int n_arrays, void* 
       }
     };
     auto cols = [&](const FftPair& io, int k, int inv) {
-      if (!gy) {
+      if (my.ns) {
+        mix_fft(dim3(nx / mw, 1, k), dim3(mix_threads(my, mw, mw)), cl, st, io, my, twy, nx, mw, mix_magic(mw), false,
+                inv != 0, 1.0);
+      } else if (!gy) {
         ((FColFn)fc->launch)(dim3(nx / cw, 1, k), dim3(cw * (ny / ce)), cl, st, io, nx, inv, twy);
       } else if (f64) {
         hipLaunchKernelGGL(gen_fft_cols_kernel<double>, dim3(nx / cw, 1, k), dim3(kGenThreads), cl, st, io, gfy,

@@ -270,7 +270,7 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
   return n % kXcds == 0 ? (b % kXcds) * (n / kXcds) + b / kXcds : b;
 }
 
-// Kinetic factors of the column pass on this thread's E points of column jx:
+// Kinetic factors of the column pass on this thread's E points t + j T of column jx:
 // the closing K of the previous sub-step (unless the state is already in
 // k-space: `kspace`) and the opening K of this one (`mid`), with the norm sums.
 // S is the norm between the two, NRM the one after both; want_s: S is asked
@@ -286,8 +286,8 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 // The uniform choices are taken around whole point loops: tested per point,
 // they put every table read in a block of its own with its own wait, a chain
 // of dependent LDS round trips.
-template <typename R, int E, int T, bool DENSE, bool IMAG, bool KYG, typename C>
-__device__ __forceinline__ void col_kinetic(C (&a)[E], int t, int nx, int jx, const double* __restrict__ td, R hp,
+template <typename R, int E, bool DENSE, bool IMAG, bool KYG, typename C>
+__device__ __forceinline__ void col_kinetic(C (&a)[E], int t, int T, int nx, int jx, const double* __restrict__ td, R hp,
                                             R hc, C kx, const C* ky, bool kspace, bool mid, bool want_s,
                                             double& s_acc, double& n_acc) {
   auto yval = [&](int j) -> C { return KYG ? ld_global(ky + t + j * T) : ky[t + j * T]; };
@@ -438,21 +438,21 @@ __device__ __forceinline__ void col_item(const InstDev& P, typename Cx<R>::T* __
   const bool want_s = mode == COL_MID_S;
   if (!DENSE || !td) {
     if (imag) {
-      col_kinetic<R, E, T, false, true, !kKy>(a, t, nx, jx, nullptr, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
+      col_kinetic<R, E, false, true, !kKy>(a, t, T, nx, jx, nullptr, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
     } else if (kspace) {  // first pass from k-space: K_cur's own tables
       const C kc = ld_global(reinterpret_cast<const C*>(P.kx[d_cur][comp]) + jx);
-      col_kinetic<R, E, T, false, false, true>(a, t, nx, jx, nullptr, hp, hc, kc,
+      col_kinetic<R, E, false, false, true>(a, t, T, nx, jx, nullptr, hp, hc, kc,
                                                reinterpret_cast<const C*>(P.ky[d_cur][comp]), true, mid, want_s,
                                                s_acc, n_acc);
     } else {
-      col_kinetic<R, E, T, false, false, !kKy>(a, t, nx, jx, nullptr, hp, hc, kx, ky, false, mid, want_s, s_acc,
+      col_kinetic<R, E, false, false, !kKy>(a, t, T, nx, jx, nullptr, hp, hc, kx, ky, false, mid, want_s, s_acc,
                                                n_acc);
     }
   } else if constexpr (DENSE) {
     if (imag)
-      col_kinetic<R, E, T, true, true, !kKy>(a, t, nx, jx, td, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
+      col_kinetic<R, E, true, true, !kKy>(a, t, T, nx, jx, td, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
     else
-      col_kinetic<R, E, T, true, false, !kKy>(a, t, nx, jx, td, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
+      col_kinetic<R, E, true, false, !kKy>(a, t, T, nx, jx, td, hp, hc, kx, ky, kspace, mid, want_s, s_acc, n_acc);
   }
   // Columns of 1024 points and more, and complex64 columns: an opaque copy of
   // t for the inverse transform and the stores, so their addresses are
@@ -706,10 +706,10 @@ __device__ __forceinline__ R fast_top(const C (&a0)[E], const C (&a1)[E], const 
 }
 
 // Points J0 <= j < J1 of a row: FAST as above, else with dense potentials and
-// coupling arrays where the slot has them.
-template <typename R, int N, int E, int T, bool FAST, int J0 = 0, int J1 = E, typename C>
-__device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const InstDev& P, const RowCoef<R>& k, int y,
-                                              int t, C py0, C py1, const C (&tx0)[E], const C (&tx1)[E],
+// coupling arrays where the slot has them (point j at base + j T of them).
+template <typename R, int E, bool FAST, int J0 = 0, int J1 = E, typename C>
+__device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const InstDev& P, const RowCoef<R>& k,
+                                              size_t base, int T, C py0, C py1, const C (&tx0)[E], const C (&tx1)[E],
                                               const C (&tex)[E]) {
   if constexpr (FAST) {
     with_variant<R>(k, fast_top<R, E, J0, J1>(a0, a1, k), [&](auto v) {
@@ -720,11 +720,10 @@ __device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const Inst
     const double* vd0 = P.v_dense[0];
     const double* vd1 = P.v_dense[1];
     const double* omd = P.coupling == 2 ? P.omega_dense : nullptr;
-    const size_t base = (size_t)y * N + t;
     R v0[M], v1[M], an[M];
 #pragma unroll
     for (int i = 0; i < M; ++i) {
-      const size_t at = base + (J0 + i) * T;
+      const size_t at = base + (size_t)((J0 + i) * T);
       v0[i] = vd0 ? (R)ld_global(vd0 + at) * k.dts : (R)0;
       v1[i] = vd1 ? (R)ld_global(vd1 + at) * k.dts : (R)0;
       an[i] = omd ? (R)ld_global(omd + at) * k.dts * (R)0.25 : (R)0;
@@ -930,7 +929,7 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
     if constexpr (GENERAL)
       pointwise_points<E, T, 0>(t, tx0, tx1, tex, px0, px1, eth, tws, [&](auto j) {
         constexpr int J = decltype(j)::v;
-        row_pointwise<R, N, E, T, false, J, J + 1>(a0, a1, P, k, y, t, py0, py1, tx0, tx1, tex);
+        row_pointwise<R, E, false, J, J + 1>(a0, a1, P, k, (size_t)y * N + t, T, py0, py1, tx0, tx1, tex);
       });
     else {
       const R top = fast_top<R, E, 0, E>(a0, a1, k);
@@ -949,11 +948,11 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   } else {
     constexpr int H = kEarlyTables ? E : E / 2;
     if constexpr (!kEarlyTables) load_x_tables<E, T, 0, H>(tx0, tx1, tex, px0, px1, eth, tws, t);
-    row_pointwise<R, N, E, T, !GENERAL, 0, H>(a0, a1, P, k, y, t, py0, py1, tx0, tx1, tex);
+    row_pointwise<R, E, !GENERAL, 0, H>(a0, a1, P, k, (size_t)y * N + t, T, py0, py1, tx0, tx1, tex);
     if constexpr (H < E) {
       __builtin_amdgcn_sched_barrier(0);
       load_x_tables<E, T, H, E>(tx0, tx1, tex, px0, px1, eth, tws, t);
-      row_pointwise<R, N, E, T, !GENERAL, H, E>(a0, a1, P, k, y, t, py0, py1, tx0, tx1, tex);
+      row_pointwise<R, E, !GENERAL, H, E>(a0, a1, P, k, (size_t)y * N + t, T, py0, py1, tx0, tx1, tex);
     }
   }
   // Large rows: the forward transform and the stores index by an opaque copy
@@ -1157,7 +1156,7 @@ __global__ __launch_bounds__(ROWS * 2 * (N / E)) void row_split_kernel(const Ins
     p1[j] = sm[N + V::at(tid + j * TP)];
   }
   const RowCoef<R> k(P, dur, lam2);
-  row_pointwise<R, N, EP, TP, !GENERAL>(p0, p1, P, k, y, tid, py0, py1, tx0, tx1, tex);
+  row_pointwise<R, EP, !GENERAL>(p0, p1, P, k, (size_t)y * N + tid, TP, py0, py1, tx0, tx1, tex);
 #pragma unroll
   for (int j = 0; j < EP; ++j) {
     sm[V::at(tid + j * TP)] = p0[j];

@@ -26,7 +26,7 @@ FLAGS = ['-O3', '-std=c++17', f'--offload-arch={ARCH}', '-fPIC', '-Wno-unused-re
          '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
          '-mllvm', '-amdgpu-kernarg-preload-count=16']
 SOURCES = ['sgpe_api.hip', 'sgpe_inst_f64.hip', 'sgpe_inst_f32.hip', 'sgpe_persist_f64.hip',
-           'sgpe_persist_f32.hip', 'sgpe_unwrap.cpp']
+           'sgpe_persist_f32.hip', 'sgpe_mixed_f64.hip', 'sgpe_mixed_f32.hip', 'sgpe_unwrap.cpp']
 
 
 def _run(cmd, verbose):
