@@ -261,13 +261,12 @@ static bool mix_fits(const MixFft& f, int batch, size_t cs, size_t lds_max) {
   return true;
 }
 
-// Threads of a workgroup of `batch` transforms (`mid` of them in the last
-// stage: rows take two components together): all inner butterflies at once,
+// Threads of a workgroup of `batch` transforms: all inner butterflies at once,
 // the outer stages in as few even rounds.
-static int mix_threads(const MixFft& f, int batch, int mid) {
+static int mix_threads(const MixFft& f, int batch) {
   int t = 64;
   for (int s = 1; s < f.ns - 1; ++s) t = std::max(t, f.st[s].nb * batch);
-  const int outer = std::max(f.st[0].nb * batch, f.st[f.ns - 1].nb * mid);
+  const int outer = std::max(f.st[0].nb, f.st[f.ns - 1].nb) * batch;
   const int rounds = (outer + kMixThreads - 1) / kMixThreads;
   t = std::max(t, (outer + rounds - 1) / rounds);
   return std::min((t + 63) / 64 * 64, kMixThreads);
@@ -737,7 +736,7 @@ static void launch_col(sgpe_plan* p, hipStream_t s, int mode, int dprev, int dcu
                        hipEvent_t e1 = nullptr) {
   if (p->mfy.ns) {
     const auto launch = p->prec == SGPE_C128 ? MixKernels<double>::col : MixKernels<float>::col;
-    launch(dim3(p->nx / p->col_w, 2, p->nlaunch), dim3(mix_threads(p->mfy, p->col_w, p->col_w)),
+    launch(dim3(p->nx / p->col_w, 2, p->nlaunch), dim3(mix_threads(p->mfy, p->col_w)),
            mix_lds(p->col_w, p->ny, csize(p->prec)), s, e0, e1, p->d_inst, p->d_run, p->mfy, p->root_y, p->col_w,
            mix_magic(p->col_w), mode, dprev, dcur);
     return;
@@ -764,9 +763,9 @@ static void launch_row(sgpe_plan* p, hipStream_t s, int dur, int first, hipEvent
                        hipEvent_t e1 = nullptr) {
   if (p->mfx.ns) {
     const auto launch = p->prec == SGPE_C128 ? MixKernels<double>::row : MixKernels<float>::row;
-    launch(dim3(p->ny / p->mix_rows, 1, p->nlaunch), dim3(mix_threads(p->mfx, 2 * p->mix_rows, p->mix_rows)),
+    launch(dim3(p->ny / p->mix_rows, 1, p->nlaunch), dim3(mix_threads(p->mfx, 2 * p->mix_rows)),
            mix_lds(2 * p->mix_rows, p->nx, csize(p->prec)), s, e0, e1, p->d_inst, p->d_run, p->mfx, p->root_x,
-           p->mix_rows, dur, first, p->col_w, p->general_row);
+           p->mix_rows, mix_magic(p->nx), dur, first, p->col_w, p->general_row);
     return;
   }
   if (p->gen_x) {
@@ -1375,7 +1374,7 @@ int sgpe_fft2(sgpe_ctx* ctx, int precision, int ny, int nx, int n_arrays, void* 
     const auto mix_fft = f64 ? MixKernels<double>::fft : MixKernels<float>::fft;
     auto rows = [&](const FftPair& io, int k, int inv, double scale) {
       if (mx.ns) {
-        mix_fft(dim3(ny / mrows, 1, k), dim3(mix_threads(mx, mrows, mrows)), rl, st, io, mx, twx, nx, mrows,
+        mix_fft(dim3(ny / mrows, 1, k), dim3(mix_threads(mx, mrows)), rl, st, io, mx, twx, nx, mrows,
                 mix_magic(mrows), true, inv != 0, scale);
       } else if (!gx) {
         ((FRowFn)fr->launch)(dim3(ny / rr, 1, k), dim3(rr * (nx / re)), rl, st, io, inv, 1, scale, twx);
@@ -1389,7 +1388,7 @@ int sgpe_fft2(sgpe_ctx* ctx, int precision, int ny, int nx, int n_arrays, void* 
     };
     auto cols = [&](const FftPair& io, int k, int inv) {
       if (my.ns) {
-        mix_fft(dim3(nx / mw, 1, k), dim3(mix_threads(my, mw, mw)), cl, st, io, my, twy, nx, mw, mix_magic(mw), false,
+        mix_fft(dim3(nx / mw, 1, k), dim3(mix_threads(my, mw)), cl, st, io, my, twy, nx, mw, mix_magic(mw), false,
                 inv != 0, 1.0);
       } else if (!gy) {
         ((FColFn)fc->launch)(dim3(nx / cw, 1, k), dim3(cw * (ny / ce)), cl, st, io, nx, inv, twy);

@@ -632,12 +632,15 @@ template <int V> struct PointVariant { static constexpr int v = V; };
 
 // Calls f(PointVariant<V>) for the variant of an instance; `top` is the
 // largest phase of this thread's points. The choice is uniform over the wave.
+// The theta-free variant is complex64's alone: there it saves 1-3 % of a batched
+// row pass, in complex128 the third way out of the branch costs more registers
+// than its arithmetic saves (32 x 256^2: 37.5 us with it, 32.3 without).
 template <typename R, class F>
 __device__ __forceinline__ void with_variant(const RowCoef<R>& k, R top, F&& f) {
   if (k.imag) {
     if (__builtin_amdgcn_ballot_w64(!(top <= (R)kSmallExp)))
       f(PointVariant<PV_IMAG>());
-    else if (k.theta)
+    else if (sizeof(R) == 8 || k.theta)
       f(PointVariant<PV_IMAG_SMALL>());
     else
       f(PointVariant<PV_IMAG_SMALL_NT>());
@@ -678,17 +681,29 @@ template <bool IMAG, typename C> __device__ __forceinline__ C pot_factor(C tx, C
     return cmul(tx, py);
 }
 
-// Points J0 <= j < J1 of a row on the fast operator path, in one variant.
-template <typename R, int V, int E, int J0, int J1, typename C>
-__device__ __forceinline__ void fast_points(C (&a0)[E], C (&a1)[E], const RowCoef<R>& k, C py0, C py1,
+// The y factor of every point of one row.
+template <typename C> struct RowFactor {
+  C v;
+  __device__ __forceinline__ C operator[](int) const { return v; }
+};
+
+// Offsets j T of a thread's points of a row.
+template <int T> struct RowStride {
+  __device__ __forceinline__ size_t operator()(int j) const { return (size_t)(j * T); }
+};
+
+// Points J0 <= j < J1 of a row on the fast operator path, in one variant. PY:
+// the points' y factors (RowFactor, or one per point).
+template <typename R, int V, int E, int J0, int J1, typename C, typename PY>
+__device__ __forceinline__ void fast_points(C (&a0)[E], C (&a1)[E], const RowCoef<R>& k, const PY& py0, const PY& py1,
                                             const C (&tx0)[E], const C (&tx1)[E], const C (&tex)[E]) {
   constexpr bool IMAG = V >= PV_IMAG_SMALL_NT;
 #pragma unroll
   for (int j = J0; j < J1; ++j) {
     R e0, e1;
     point_phases<R>(a0[j], a1[j], k, &e0, &e1);
-    point_ops<R, V>(a0[j], a1[j], e0, e1, k.sc, k.ca, k.cb, pot_factor<IMAG>(tx0[j], py0),
-                    pot_factor<IMAG>(tx1[j], py1), tex[j]);
+    point_ops<R, V>(a0[j], a1[j], e0, e1, k.sc, k.ca, k.cb, pot_factor<IMAG>(tx0[j], py0[j]),
+                    pot_factor<IMAG>(tx1[j], py1[j]), tex[j]);
   }
 }
 
@@ -706,11 +721,11 @@ __device__ __forceinline__ R fast_top(const C (&a0)[E], const C (&a1)[E], const 
 }
 
 // Points J0 <= j < J1 of a row: FAST as above, else with dense potentials and
-// coupling arrays where the slot has them (point j at base + j T of them).
-template <typename R, int E, bool FAST, int J0 = 0, int J1 = E, typename C>
+// coupling arrays where the slot has them (point j at base + offset(j) of them).
+template <typename R, int E, bool FAST, int J0 = 0, int J1 = E, typename C, typename PY, typename At>
 __device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const InstDev& P, const RowCoef<R>& k,
-                                              size_t base, int T, C py0, C py1, const C (&tx0)[E], const C (&tx1)[E],
-                                              const C (&tex)[E]) {
+                                              size_t base, const At& offset, const PY& py0, const PY& py1, const C (&tx0)[E],
+                                              const C (&tx1)[E], const C (&tex)[E]) {
   if constexpr (FAST) {
     with_variant<R>(k, fast_top<R, E, J0, J1>(a0, a1, k), [&](auto v) {
       fast_points<R, decltype(v)::v, E, J0, J1>(a0, a1, k, py0, py1, tx0, tx1, tex);
@@ -723,7 +738,7 @@ __device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const Inst
     R v0[M], v1[M], an[M];
 #pragma unroll
     for (int i = 0; i < M; ++i) {
-      const size_t at = base + (size_t)((J0 + i) * T);
+      const size_t at = base + offset(J0 + i);
       v0[i] = vd0 ? (R)ld_global(vd0 + at) * k.dts : (R)0;
       v1[i] = vd1 ? (R)ld_global(vd1 + at) * k.dts : (R)0;
       an[i] = omd ? (R)ld_global(omd + at) * k.dts * (R)0.25 : (R)0;
@@ -750,8 +765,8 @@ __device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const Inst
             b = u.y;
           }
         }
-        const C f0 = vd0 ? phase_op<R, IMAG, SMALL>(v0[i]) : pot_factor<IMAG>(tx0[j], py0);
-        const C f1 = vd1 ? phase_op<R, IMAG, SMALL>(v1[i]) : pot_factor<IMAG>(tx1[j], py1);
+        const C f0 = vd0 ? phase_op<R, IMAG, SMALL>(v0[i]) : pot_factor<IMAG>(tx0[j], py0[j]);
+        const C f1 = vd1 ? phase_op<R, IMAG, SMALL>(v1[i]) : pot_factor<IMAG>(tx1[j], py1[j]);
         R e0, e1;
         point_phases<R>(a0[j], a1[j], k, &e0, &e1);
         point_ops<R, V>(a0[j], a1[j], e0, e1, k.sc, a, b, f0, f1, tex[j]);
@@ -924,12 +939,13 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   // halves, which already fit 3 waves per SIMD (point by point would only
   // add latency).
   const RowCoef<R> k(P, dur, lam2);
+  const RowFactor<C> fy0{py0}, fy1{py1};
   if constexpr (E >= 8 && sizeof(C) == 16) {
     load_x_tables<E, T, 0, 1>(tx0, tx1, tex, px0, px1, eth, tws, t);
     if constexpr (GENERAL)
       pointwise_points<E, T, 0>(t, tx0, tx1, tex, px0, px1, eth, tws, [&](auto j) {
         constexpr int J = decltype(j)::v;
-        row_pointwise<R, E, false, J, J + 1>(a0, a1, P, k, (size_t)y * N + t, T, py0, py1, tx0, tx1, tex);
+        row_pointwise<R, E, false, J, J + 1>(a0, a1, P, k, (size_t)y * N + t, RowStride<T>(), fy0, fy1, tx0, tx1, tex);
       });
     else {
       const R top = fast_top<R, E, 0, E>(a0, a1, k);
@@ -941,18 +957,18 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
       with_variant<R>(k, top, [&](auto v) {
         pointwise_points<E, T, 0>(t, tx0, tx1, tex, px0, px1, eth, tws, [&](auto j) {
           constexpr int J = decltype(j)::v;
-          fast_points<R, decltype(v)::v, E, J, J + 1>(a0, a1, k, py0, py1, tx0, tx1, tex);
+          fast_points<R, decltype(v)::v, E, J, J + 1>(a0, a1, k, fy0, fy1, tx0, tx1, tex);
         });
       });
     }
   } else {
     constexpr int H = kEarlyTables ? E : E / 2;
     if constexpr (!kEarlyTables) load_x_tables<E, T, 0, H>(tx0, tx1, tex, px0, px1, eth, tws, t);
-    row_pointwise<R, E, !GENERAL, 0, H>(a0, a1, P, k, (size_t)y * N + t, T, py0, py1, tx0, tx1, tex);
+    row_pointwise<R, E, !GENERAL, 0, H>(a0, a1, P, k, (size_t)y * N + t, RowStride<T>(), fy0, fy1, tx0, tx1, tex);
     if constexpr (H < E) {
       __builtin_amdgcn_sched_barrier(0);
       load_x_tables<E, T, H, E>(tx0, tx1, tex, px0, px1, eth, tws, t);
-      row_pointwise<R, E, !GENERAL, H, E>(a0, a1, P, k, (size_t)y * N + t, T, py0, py1, tx0, tx1, tex);
+      row_pointwise<R, E, !GENERAL, H, E>(a0, a1, P, k, (size_t)y * N + t, RowStride<T>(), fy0, fy1, tx0, tx1, tex);
     }
   }
   // Large rows: the forward transform and the stores index by an opaque copy
@@ -1156,7 +1172,8 @@ __global__ __launch_bounds__(ROWS * 2 * (N / E)) void row_split_kernel(const Ins
     p1[j] = sm[N + V::at(tid + j * TP)];
   }
   const RowCoef<R> k(P, dur, lam2);
-  row_pointwise<R, EP, !GENERAL>(p0, p1, P, k, (size_t)y * N + tid, TP, py0, py1, tx0, tx1, tex);
+  row_pointwise<R, EP, !GENERAL>(p0, p1, P, k, (size_t)y * N + tid, RowStride<TP>(), RowFactor<C>{py0},
+                                 RowFactor<C>{py1}, tx0, tx1, tex);
 #pragma unroll
   for (int j = 0; j < EP; ++j) {
     sm[V::at(tid + j * TP)] = p0[j];

@@ -10,8 +10,8 @@
 //     pointwise block, then the adjoint stages back in reverse order:
 // the second transform is the conjugate transpose of the first, stage by
 // stage, so it reads the same twiddle table, its first stage works on the very
-// points a thread holds after the last stage of the first transform (which,
-// pointwise block and all, is then one read and one write of LDS in place), and
+// points a thread holds after the last stage of the first transform (in place in
+// LDS; the column pass applies its factors between the two in registers), and
 // its last stage writes to global memory what stage 0 read. Against keeping the
 // data in LDS throughout, with one stage per prime power, twiddles gathered from
 // global memory and two LDS buffers (sgpe_generic.h), a 600-point pass makes 4
@@ -21,7 +21,7 @@
 // stage is an LDS round trip and a barrier), by LDS and vector instructions in
 // batches. Measured (dispatch times, us, sgpe_generic.h -> here): 600 x 480
 // complex128 column 30.9 -> 18.5, row 23.8 -> 15.6; 1000^2 complex64 column 52.1
-// -> 22.2, row 34.7 -> 29.3; 1536^2 complex128 column 168 -> 67, row 190 -> 65.
+// -> 22.2, row 34.7 -> 21.7; 1536^2 complex128 column 168 -> 67, row 190 -> 92.
 #pragma once
 
 #include <type_traits>
@@ -34,7 +34,7 @@ constexpr int kMixMaxStages = 5;
 constexpr int kMixMaxLen = 2048;
 constexpr int kMixMinLen = 32;
 constexpr int kMixMaxRadix = 16;
-constexpr int kMixMidRadix = 10;  // last stage: holds its twiddles and, in the row pass, both components
+constexpr int kMixMidRadix = 10;  // last stage: holds its twiddles
 constexpr int kMixThreads = 512;  // most threads of a workgroup
 
 // One stage: radix, span (product of the radices before it), butterflies,
@@ -475,13 +475,24 @@ __global__ __launch_bounds__(kMixThreads) void mix_col_pass_kernel(const InstDev
 }
 
 // -------------------------------------------------------------- row pass
+
+// Offsets of a thread's points i0 + j step in an array of `end`; point 0 stands
+// in for those past the end.
+struct PointsAt {
+  int i0, step, end;
+  __device__ __forceinline__ size_t operator()(int j) const {
+    const int i = i0 + j * step;
+    return (size_t)(i < end ? i : i0);
+  }
+};
+
 // `rows` rows (both components) of slot blockIdx.z, as row_pass_kernel.
 // LDS: [rows][2][n] data, [n] twiddles. GENERAL as there.
 template <typename R, bool GENERAL>
 __global__ __launch_bounds__(kMixThreads) void mix_row_pass_kernel(const InstDev* __restrict__ insts,
                                                                    RunDev* __restrict__ runs, MixFft f,
                                                                    const typename Cx<R>::T* __restrict__ tw, int rows,
-                                                                   int dur, int first_sub, int col_w) {
+                                                                   unsigned div_n, int dur, int first_sub, int col_w) {
   typedef typename Cx<R>::T C;
   extern __shared__ double smem[];
   const int inst = blockIdx.z;
@@ -517,70 +528,80 @@ __global__ __launch_bounds__(kMixThreads) void mix_row_pass_kernel(const InstDev
   const double lam2 = P.atom_num / (P.dv_r * (double)N * (double)ny * nrm);
   mix_inner<true>(f, x);
 
-  // Last stage of both components of a row, pointwise block, adjoint last
-  // stage.
-  const double* vd0 = P.v_dense[0];
-  const double* vd1 = P.v_dense[1];
-  const C* px0 = vd0 ? tw : reinterpret_cast<const C*>(P.px[dur][0]);  // absent: any n - 1 entries stand in
-  const C* px1 = vd1 ? tw : reinterpret_cast<const C*>(P.px[dur][1]);
-  const C* eth = reinterpret_cast<const C*>(P.etheta);
-  const RowCoef<R> k(P, dur, lam2);
+  // Last stage in place, pointwise block over all points of the rows, two per
+  // thread at a time (four: 233 registers, 10-35 % slower), adjoint last stage in place. With the block inside the
+  // last stage (as the column pass has it) a thread held both components of up
+  // to ten points: 256 registers, a third of the threads idle, and for dense
+  // operators 30 KB of straight-line code per radix, whose fetching took longer
+  // than its work on small grids. 96 x 100 complex128, dense: 20-28 -> 9 us;
+  // 1000^2 dense 85-93 -> 46 us; 1000^2 fast path 44 -> 36 us (complex128) and 30
+  // -> 22 us (complex64); 1536^2 complex128 is the exception (65 -> 92 us).
   const MixStage& st = f.st[f.ns - 1];
-  const int items = st.nb * rows;
+  const int items = st.nb * x.batch;
   mix_radix<kMixMidRadix>(st.radix, [&](auto rr) {
     constexpr int E = decltype(rr)::v;
-    // All waves of the workgroup stay in the loop together only as far as
-    // their own items go: no barrier inside.
     for (int w = threadIdx.x; w < items; w += blockDim.x) {
-      const int row = mix_div(w, st.nb, st.div_nb);
-      const int v = w - row * st.nb;
-      const int y = y0 + row;
-      const C* wk = x.tw + st.off + v * (E - 1);
-      C a0[E], a1[E];
+      int m, v;
+      x.item(st, w, &m, &v);
+      C b[E];
 #pragma unroll
-      for (int r = 0; r < E; ++r) {
-        a0[r] = x.at(2 * row, v + r * st.nb);
-        a1[r] = x.at(2 * row + 1, v + r * st.nb);
-      }
-      mix_twiddle<E, true>(a0, wk);
-      mix_twiddle<E, true>(a1, wk);
-      mix_dft<E, true>(a0);
-      mix_dft<E, true>(a1);
-      const C py0 = vd0 ? C{1, 0} : ld_global(reinterpret_cast<const C*>(P.py[dur][0]) + y);
-      const C py1 = vd1 ? C{1, 0} : ld_global(reinterpret_cast<const C*>(P.py[dur][1]) + y);
-      C tx0[E], tx1[E], tex[E];
-      auto tables = [&](auto j0, auto j1) {
+      for (int r = 0; r < E; ++r) b[r] = x.at(m, v + r * st.nb);
+      mix_twiddle<E, true>(b, x.tw + st.off + v * (E - 1));  // k = v: the span is n / radix
+      mix_dft<E, true>(b);
 #pragma unroll
-        for (int r = decltype(j0)::v; r < decltype(j1)::v; ++r) {
-          const int i = v + r * st.nb;
-          tx0[r] = ld_global(px0 + (vd0 ? 0 : i));
-          tx1[r] = ld_global(px1 + (vd1 ? 0 : i));
-          tex[r] = ld_global(eth + i);
-        }
-      };
-      // In two halves, as row_item does, to bound the registers.
-      constexpr int H = E <= 3 ? E : (E + 1) / 2;
-      const size_t base = (size_t)y * N + v;
-      tables(PointVariant<0>(), PointVariant<H>());
-      row_pointwise<R, E, !GENERAL, 0, H>(a0, a1, P, k, base, st.nb, py0, py1, tx0, tx1, tex);
-      if constexpr (H < E) {
-        __builtin_amdgcn_sched_barrier(0);
-        tables(PointVariant<H>(), PointVariant<E>());
-        row_pointwise<R, E, !GENERAL, H, E>(a0, a1, P, k, base, st.nb, py0, py1, tx0, tx1, tex);
-      }
-      // The twiddles again from LDS rather than held since the first use.
-      int vo = v;
-      asm volatile("" : "+v"(vo));
-      wk = x.tw + st.off + vo * (E - 1);
-      mix_dft<E, false>(a0);
-      mix_dft<E, false>(a1);
-      mix_twiddle<E, false>(a0, wk);
-      mix_twiddle<E, false>(a1, wk);
+      for (int r = 0; r < E; ++r) x.at(m, v + r * st.nb) = b[r];
+    }
+  });
+  const double* vd0 = P.v_dense[0];
+  const double* vd1 = P.v_dense[1];
+  const C* px0 = vd0 ? nullptr : reinterpret_cast<const C*>(P.px[dur][0]);
+  const C* px1 = vd1 ? nullptr : reinterpret_cast<const C*>(P.px[dur][1]);
+  const C* qy0 = vd0 ? nullptr : reinterpret_cast<const C*>(P.py[dur][0]);
+  const C* qy1 = vd1 ? nullptr : reinterpret_cast<const C*>(P.py[dur][1]);
+  const C* eth = reinterpret_cast<const C*>(P.etheta);
+  const RowCoef<R> k(P, dur, lam2);
+  const int points = rows * N;
+  __syncthreads();
+  for (int i0 = threadIdx.x; i0 < points; i0 += 2 * (int)blockDim.x) {
+    const PointsAt offset{i0, (int)blockDim.x, points};
+    C a0[2], a1[2], tx0[2], tx1[2], tex[2], py0[2], py1[2];
+    int at[2];
 #pragma unroll
-      for (int r = 0; r < E; ++r) {
-        x.at(2 * row, v + r * st.nb) = a0[r];
-        x.at(2 * row + 1, v + r * st.nb) = a1[r];
-      }
+    for (int j = 0; j < 2; ++j) {
+      const int i = (int)offset(j);
+      const int row = mix_div(i, N, div_n), xx = i - row * N;
+      at[j] = i + row * N;  // (2 row) n + xx
+      tx0[j] = px0 ? ld_global(px0 + xx) : C{1, 0};
+      tx1[j] = px1 ? ld_global(px1 + xx) : C{1, 0};
+      tex[j] = ld_global(eth + xx);
+      py0[j] = qy0 ? ld_global(qy0 + y0 + row) : C{1, 0};
+      py1[j] = qy1 ? ld_global(qy1 + y0 + row) : C{1, 0};
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      a0[j] = x.lds[at[j]];
+      a1[j] = x.lds[at[j] + N];
+    }
+    row_pointwise<R, 2, !GENERAL>(a0, a1, P, k, (size_t)y0 * N, offset, py0, py1, tx0, tx1, tex);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      x.lds[at[j]] = a0[j];
+      x.lds[at[j] + N] = a1[j];
+    }
+  }
+  __syncthreads();
+  mix_radix<kMixMidRadix>(st.radix, [&](auto rr) {
+    constexpr int E = decltype(rr)::v;
+    for (int w = threadIdx.x; w < items; w += blockDim.x) {
+      int m, v;
+      x.item(st, w, &m, &v);
+      C b[E];
+#pragma unroll
+      for (int r = 0; r < E; ++r) b[r] = x.at(m, v + r * st.nb);
+      mix_dft<E, false>(b);
+      mix_twiddle<E, false>(b, x.tw + st.off + v * (E - 1));
+#pragma unroll
+      for (int r = 0; r < E; ++r) x.at(m, v + r * st.nb) = b[r];
     }
   });
   mix_inner_adj<false>(f, x);
@@ -652,7 +673,7 @@ template <typename R> struct MixKernels {
   static void col(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const InstDev* i, RunDev* r,
                   const MixFft& f, const void* tw, int w, unsigned div_w, int mode, int dp, int dc);
   static void row(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const InstDev* i, RunDev* r,
-                  const MixFft& f, const void* tw, int rows, int dur, int first, int col_w, bool general);
+                  const MixFft& f, const void* tw, int rows, unsigned div_n, int dur, int first, int col_w, bool general);
   static void fft(dim3 g, dim3 b, size_t l, hipStream_t s, FftPair io, const MixFft& f, const void* tw, int nx,
                   int batch, unsigned div_batch, bool rows, bool inv, double scale);
   static const void* kernel(int which);

@@ -23,13 +23,13 @@ void MixKernels<R>::col(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, 
 
 template <typename R>
 void MixKernels<R>::row(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const InstDev* i,
-                        RunDev* r, const MixFft& f, const void* tw, int rows, int dur, int first, int col_w,
-                        bool general) {
+                        RunDev* r, const MixFft& f, const void* tw, int rows, unsigned div_n, int dur, int first,
+                        int col_w, bool general) {
   const typename Cx<R>::T* t = (const typename Cx<R>::T*)tw;
   if (general)
-    SGPE_MIX_LAUNCH((mix_row_pass_kernel<R, true>), i, r, f, t, rows, dur, first, col_w);
+    SGPE_MIX_LAUNCH((mix_row_pass_kernel<R, true>), i, r, f, t, rows, div_n, dur, first, col_w);
   else
-    SGPE_MIX_LAUNCH((mix_row_pass_kernel<R, false>), i, r, f, t, rows, dur, first, col_w);
+    SGPE_MIX_LAUNCH((mix_row_pass_kernel<R, false>), i, r, f, t, rows, div_n, dur, first, col_w);
 }
 
 template <typename R>
