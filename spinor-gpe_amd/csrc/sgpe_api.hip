@@ -782,7 +782,8 @@ static void launch_row(sgpe_plan* p, hipStream_t s, int dur, int first, hipEvent
   const size_t lds = row_pass_lds(p->row_e, p->row_rows, p->nx, csize(p->prec));
   dim3 grid(p->ny / std::abs(p->row_rows), 1, p->nlaunch), block(row_block_threads(p->row_e, p->row_rows, p->nx));
   ((RowFn)(p->general_row ? p->row->launch_g : p->row->launch))(grid, block, lds, s, e0, e1, p->d_inst, p->d_run,
-                                                                direct_state(p), p->ny, p->tw_x, dur, first, p->col_w,
+                                                                direct_state(p), p->h_inst[0].part, p->ny, p->tw_x, dur,
+                                                                first, p->col_w,
                                                                 p->row_stream);
 }
 

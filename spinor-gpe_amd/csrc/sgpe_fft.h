@@ -161,10 +161,28 @@ template <int ELEM_BYTES> struct SwzView {
   static constexpr int span(int n) { return n; }
 };
 
+// Twiddles of one stage held by a thread: (E / R) butterflies of R - 1.
+template <int N, int E, int L, typename C> struct StageTwiddles {
+  static constexpr int R = (N / L >= E) ? E : N / L;
+  static constexpr bool kAny = L > 1 && L < N;
+  C w[kAny ? (E / R) * (R - 1) : 1];
+  __device__ __forceinline__ void load(int t, const C* __restrict__ tw) {
+    if constexpr (kAny) {
+#pragma unroll
+      for (int u = 0; u < E / R; ++u) {
+        const int k = (t + u * (N / E)) & (L - 1);
+#pragma unroll
+        for (int r = 1; r < R; ++r) w[u * (R - 1) + r - 1] = ld_global(tw + (L - 1) + k * (R - 1) + (r - 1));
+      }
+    }
+  }
+};
+
 // One Stockham stage. Non-final stages write their outputs to LDS; the final
-// stage leaves output Y[t + j*T] in a[j].
-template <int N, int E, int R, int L, bool INV, bool LAST, class V, typename C>
-__device__ __forceinline__ void fft_stage(C (&a)[E], int t, const C* tw, C* lds) {
+// stage leaves output Y[t + j*T] in a[j]. PRE: the twiddles are in w, else they
+// are read from tw.
+template <int N, int E, int R, int L, bool INV, bool LAST, class V, bool PRE = false, typename C>
+__device__ __forceinline__ void fft_stage(C (&a)[E], int t, const C* tw, C* lds, const C* w_pre = nullptr) {
   constexpr int T = N / E;
   constexpr int U = E / R;
   C out[LAST ? E : 1];
@@ -179,7 +197,7 @@ __device__ __forceinline__ void fft_stage(C (&a)[E], int t, const C* tw, C* lds)
       const C* wk = tw + (L - 1) + k * (R - 1) - 1;
 #pragma unroll
       for (int r = 1; r < R; ++r) {
-        C w = wk[r];
+        C w = PRE ? w_pre[u * (R - 1) + r - 1] : wk[r];
         if (INV) w.y = -w.y;
         b[r] = cmul(b[r], w);
       }
@@ -273,6 +291,49 @@ __device__ __forceinline__ void fft_run2_db(C (&a)[E], C (&b)[E], int t, const C
       b[j] = l1[V::at(t + j * T)];
     }
     fft_run2_db<N, E, INV, V, WAVE, L * R>(a, b, t, tw, m0, m1, l0, l1);
+  }
+}
+
+// fft_run and fft_run2 with the twiddle table in global memory: each stage's
+// twiddles are loaded into registers before the exchange ahead of it, so that
+// their latency passes during the exchange instead of after it. w holds those
+// of the stage of span L (L = 1 needs none).
+template <int N, int E, bool INV, class V, bool WAVE = false, int L = 1, typename C>
+__device__ __forceinline__ void fft_run_pre(C (&a)[E], int t, const C* tw, C* lds,
+                                            const StageTwiddles<N, E, L, C>& w) {
+  constexpr int R = StageTwiddles<N, E, L, C>::R;
+  constexpr bool LAST = (L * R == N);
+  constexpr int T = N / E;
+  StageTwiddles<N, E, L * R, C> next;
+  next.load(t, tw);
+  fft_stage<N, E, R, L, INV, LAST, V, true>(a, t, tw, lds, w.w);
+  if constexpr (!LAST) {
+    exchange_sync<WAVE>();
+#pragma unroll
+    for (int j = 0; j < E; ++j) a[j] = lds[V::at(t + j * T)];
+    exchange_sync<WAVE>();
+    fft_run_pre<N, E, INV, V, WAVE, L * R>(a, t, tw, lds, next);
+  }
+}
+template <int N, int E, bool INV, class V, bool WAVE = false, int L = 1, typename C>
+__device__ __forceinline__ void fft_run2_pre(C (&a)[E], C (&b)[E], int t, const C* tw, C* lds0, C* lds1,
+                                             const StageTwiddles<N, E, L, C>& w) {
+  constexpr int R = StageTwiddles<N, E, L, C>::R;
+  constexpr bool LAST = (L * R == N);
+  constexpr int T = N / E;
+  fft_stage<N, E, R, L, INV, LAST, V, true>(a, t, tw, lds0, w.w);
+  StageTwiddles<N, E, L * R, C> next;
+  next.load(t, tw);
+  fft_stage<N, E, R, L, INV, LAST, V, true>(b, t, tw, lds1, w.w);
+  if constexpr (!LAST) {
+    exchange_sync<WAVE>();
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      a[j] = lds0[V::at(t + j * T)];
+      b[j] = lds1[V::at(t + j * T)];
+    }
+    exchange_sync<WAVE>();
+    fft_run2_pre<N, E, INV, V, WAVE, L * R>(a, b, t, tw, lds0, lds1, next);
   }
 }
 

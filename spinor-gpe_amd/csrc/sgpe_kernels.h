@@ -253,6 +253,41 @@ __device__ __forceinline__ double wave_sum_strided(const double* __restrict__ p,
   return v;
 }
 
+// The same sum with the loads of the first 256 entries issued by the
+// constructor and the rest done by sum(): a row pass issues them ahead of its
+// state loads. Loads return in order, so the norm, its reduction across the
+// lanes, the division and the square root then finish while the state is still
+// on its way; loaded after the state, all of it came on top. Same order of
+// additions, same result.
+struct PartSum {
+  const double* __restrict__ p;
+  int n;
+  double e[4];
+  __device__ __forceinline__ PartSum(const double* __restrict__ part, int count) : p(part), n(count) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) e[k] = ld_global(p + (lane + 64 * k < n ? lane + 64 * k : 0));
+  }
+  __device__ __forceinline__ double sum() const {
+    const int lane = threadIdx.x & 63;
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (lane + 64 * k < n) v += e[k];
+    for (int i = lane + 256; i < n; i += 4 * 64) {
+      double f[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) f[k] = i + 64 * k < n ? ld_global(p + i + 64 * k) : 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (i + 64 * k < n) v += f[k];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+  }
+};
+
 template <typename R> __device__ __forceinline__ double norm2d(typename Cx<R>::T a) {
   double x = (double)a.x, y = (double)a.y;
   return x * x + y * y;
@@ -427,7 +462,12 @@ __device__ __forceinline__ void col_item(const InstDev& P, typename Cx<R>::T* __
 
   if (!kspace) {
     if constexpr (kWave && (kTw || kKy)) __syncthreads();  // publishes the staged tables
-    fft_run<N, E, false, V, kWave>(a, t, tw, lds);
+    if constexpr (kTw) {
+      fft_run<N, E, false, V, kWave>(a, t, tw, lds);
+    } else {
+      const StageTwiddles<N, E, 1, C> none{};
+      fft_run_pre<N, E, false, V, kWave>(a, t, tw, lds, none);
+    }
   } else {
     __syncthreads();  // publishes the staged tables
   }
@@ -461,7 +501,14 @@ __device__ __forceinline__ void col_item(const InstDev& P, typename Cx<R>::T* __
   // registers, 8 waves per SIMD instead of 5).
   int tf = t;
   if constexpr (N >= 1024 || sizeof(C) == 8) asm volatile("" : "+v"(tf));
-  if (mid) fft_run<N, E, true, V, kWave>(a, tf, tw, lds);
+  if (mid) {
+    if constexpr (kTw) {
+      fft_run<N, E, true, V, kWave>(a, tf, tw, lds);
+    } else {
+      const StageTwiddles<N, E, 1, C> none{};
+      fft_run_pre<N, E, true, V, kWave>(a, tf, tw, lds, none);
+    }
+  }
   if constexpr ((CM & CM_STORE) != 0) {
 #pragma unroll
     for (int j = 0; j < E; ++j) cb.store<C>(cbase + (uint32_t)((tf + j * T) * nx * sizeof(C)), a[j]);
@@ -830,10 +877,11 @@ __device__ __forceinline__ void record_pops(const InstDev& P, double* pops, int 
 // every global load of the prologue has been issued; false drops the block.
 // GENERAL: some slot has a dense potential or a coupling array; otherwise
 // every slot takes the separable fast path.
-template <typename R, int N, int E, int ROWS, bool GENERAL, int CM, class Gate>
+// HELD: see row_pass_kernel.
+template <typename R, int N, int E, int ROWS, bool GENERAL, int CM, bool HELD = false, class Gate>
 __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __restrict__ psi, int ny,
-                                         const typename Cx<R>::T* __restrict__ tws, int dur, int col_w, int stream,
-                                         int blk, double* smem, Gate gate) {
+                                         const double* __restrict__ part, const typename Cx<R>::T* __restrict__ tws,
+                                         int dur, int col_w, int stream, int blk, double* smem, Gate gate) {
   typedef typename Cx<R>::T C;
   typedef SwzView<sizeof(C)> V;
   constexpr int T = N / E;
@@ -856,9 +904,10 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   C* lds0 = sm + (size_t)row * 2 * N;
   C* lds1 = lds0 + N;
 
-  // Global loads first: the two rows, the twiddles (held in registers until
-  // they are stored to LDS) and the norm partials; the kernel then waits for
+  // Global loads first: the norm partials, the two rows and the twiddles (held
+  // in registers until they are stored to LDS); the kernel then waits for
   // memory once.
+  const PartSum psum(part + PART_NRM * nt2, CM ? 0 : nt2);
   C a0[E], a1[E];
   // CM: as in col_item; element (comp, y, x) at byte ((comp ny + y) N + x) sizeof(C)
   const CoherentBuf cb(psi, CM ? (uint32_t)(2 * (size_t)ny * N * sizeof(C)) : 0u);
@@ -908,21 +957,23 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   // Real-space normalization (tensor_tools.py:301-305) from the column
   // pass's k-space sums by Parseval: sum_r |IDFT2 v|^2 = Nx Ny sum_k |v|^2.
   // Every wave sums all partials itself (same order in every wave and
-  // block: no barrier, deterministic); the loads join the ones above. The
-  // twiddles stored here are published by the transform's first barrier
+  // block: no barrier, deterministic), loaded ahead of the rows. The twiddles stored here are published by the transform's first barrier
   // (its first stage uses none).
-  const double* part = P.part;
-  double nrm[1] = {wave_sum_strided<(CM & CM_LOAD) != 0>(part + PART_NRM * nt2, nt2)};
+  const double nrm = CM ? wave_sum_strided<(CM & CM_LOAD) != 0>(part + PART_NRM * nt2, nt2) : psum.sum();
   const C* tw = stw.store(sm + ROWS * 2 * N);
   if constexpr (kWave && kTw) __syncthreads();  // publishes the twiddles staged by every wave
-  const double lam2 = P.atom_num / (P.dv_r * (double)N * (double)ny * nrm[0]);
+  const double lam2 = P.atom_num / (P.dv_r * (double)N * (double)ny * nrm);
 
   C* const alt0 = sm + ROWS * 2 * N + (kTw ? N : 0) + (size_t)row * 2 * N;
   C* const alt1 = alt0 + N;
   if constexpr (kDb)
     fft_run2_db<N, E, true, V, kWave>(a0, a1, t, tw, lds0, lds1, alt0, alt1);
-  else
+  else if constexpr (kTw) {
     fft_run2<N, E, true, V, kWave>(a0, a1, t, tw, lds0, lds1);
+  } else {
+    const StageTwiddles<N, E, 1, C> none{};
+    fft_run2_pre<N, E, true, V, kWave>(a0, a1, t, tw, lds0, lds1, none);
+  }
 
   // The x-table values of this thread's points (an absent potential table
   // is stood in for by the global twiddle table: N entries, unused). Radix
@@ -983,7 +1034,7 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   // the CUs' slots already, only the recomputation remains (+2 %).
   constexpr size_t kLdsWg = kData * (kDb ? 2 : 1) + (kTw ? (size_t)N * sizeof(C) : 0);
   constexpr int kLdsWaves = (int)(kLdsBytes / kLdsWg) * ((ROWS * T + 63) / 64) / 4;
-  constexpr bool kOpaque = N >= 2048 || (N >= 1024 && kLdsWaves >= 3);
+  constexpr bool kOpaque = HELD ? false : N >= 2048 || (N >= 1024 && kLdsWaves >= 3);
   int tf = t;
   if constexpr (kOpaque) asm volatile("" : "+v"(tf));
   // The forward transform starts on the buffer pair the inverse one read
@@ -992,8 +1043,12 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
     fft_run2_db<N, E, false, V, kWave>(a0, a1, tf, tw, alt0, alt1, lds0, lds1);
   else if constexpr (kDb)
     fft_run2_db<N, E, false, V, kWave>(a0, a1, tf, tw, lds0, lds1, alt0, alt1);
-  else
+  else if constexpr (kTw) {
     fft_run2<N, E, false, V, kWave>(a0, a1, tf, tw, lds0, lds1);
+  } else {
+    const StageTwiddles<N, E, 1, C> none{};
+    fft_run2_pre<N, E, false, V, kWave>(a0, a1, tf, tw, lds0, lds1, none);
+  }
   if constexpr ((CM & CM_STORE) != 0) {
 #pragma unroll
     for (int j = 0; j < E; ++j) {
@@ -1026,10 +1081,17 @@ template <typename R, int N, int E, int ROWS> constexpr int row_min_waves() {
   return E >= 8 && cs == 16 && waves >= 2 ? 2 : 1;
 }
 
-template <typename R, int N, int E, int ROWS, bool GENERAL>
+// HELD: for launches of at most one workgroup per CU, where registers limit
+// nothing: addresses and twiddles kept from the inverse
+// transform to the forward one (at the price of a few spills). Complex128
+// 2048-point rows, 256 of them: 21.3 us
+// instead of 24.7; with 2048 of them it would be 98 instead of 79.
+constexpr int kCus = 256;
+template <typename R, int N, int E> constexpr bool row_has_held() { return sizeof(R) == 8 && N == 2048 && E == 8; }
+template <typename R, int N, int E, int ROWS, bool GENERAL, bool HELD = false>
 __global__ __launch_bounds__(ROWS*(N / E), (row_min_waves<R, N, E, ROWS>())) void row_pass_kernel(const InstDev* __restrict__ insts,
                                                                 RunDev* __restrict__ runs, void* direct_psi,
-                                                                int direct_n,
+                                                                const double* direct_part, int direct_n,
                                                                 const typename Cx<R>::T* __restrict__ tws,
                                                                 int dur, int first_sub, int col_w, int stream) {
   typedef typename Cx<R>::T C;
@@ -1037,7 +1099,7 @@ __global__ __launch_bounds__(ROWS*(N / E), (row_min_waves<R, N, E, ROWS>())) voi
   const int inst = blockIdx.z;
   RunDev& run = runs[inst];
   const InstDev& P = insts[inst];
-  // State address and column length: kernel arguments for a single-slot
+  // State and partial sums' addresses and column length: kernel arguments for a single-slot
   // plan (loads first, active flag checked after them), else read together
   // with the active flag (one round of scalar loads before the state loads).
   const bool direct = direct_psi != nullptr;
@@ -1065,7 +1127,7 @@ __global__ __launch_bounds__(ROWS*(N / E), (row_min_waves<R, N, E, ROWS>())) voi
     }
     return true;
   };
-  row_item<R, N, E, ROWS, GENERAL, 0>(P, psi, ny, tws, dur, col_w, stream, blockIdx.x, smem, gate);
+  row_item<R, N, E, ROWS, GENERAL, 0, HELD>(P, psi, ny, direct ? direct_part : P.part, tws, dur, col_w, stream, blockIdx.x, smem, gate);
 }
 
 // Row pass with the two components on separate waves (the split layout):
@@ -1082,7 +1144,7 @@ __global__ __launch_bounds__(ROWS*(N / E), (row_min_waves<R, N, E, ROWS>())) voi
 template <typename R, int N, int E, int ROWS, bool GENERAL>
 __global__ __launch_bounds__(ROWS * 2 * (N / E)) void row_split_kernel(const InstDev* __restrict__ insts,
                                                                        RunDev* __restrict__ runs, void* direct_psi,
-                                                                       int direct_n,
+                                                                       const double* direct_part, int direct_n,
                                                                        const typename Cx<R>::T* __restrict__ tws,
                                                                        int dur, int first_sub, int col_w, int stream) {
   typedef typename Cx<R>::T C;
@@ -1112,6 +1174,8 @@ __global__ __launch_bounds__(ROWS * 2 * (N / E)) void row_split_kernel(const Ins
   C* const row = psi + ((size_t)comp * ny + y) * N;
   constexpr size_t kData = (size_t)ROWS * 2 * N * sizeof(C);
   constexpr bool kTw = tw_in_lds(kData, N, sizeof(C));
+  const int nt2 = 2 * (N / col_w);
+  const PartSum psum((direct ? direct_part : P.part) + PART_NRM * nt2, nt2);  // ahead of the state, see PartSum
   C a[E];
   if (stream) {
 #pragma unroll
@@ -1142,7 +1206,6 @@ __global__ __launch_bounds__(ROWS * 2 * (N / E)) void row_split_kernel(const Ins
   }
   // Block 0 of the first sub-step records the previous full step's
   // populations and counts the step; the state leaves in hybrid form.
-  const int nt2 = 2 * (N / col_w);
   if (blockIdx.x == 0) {
     if (first_sub) {
       const int step = run.step;
@@ -1152,7 +1215,7 @@ __global__ __launch_bounds__(ROWS * 2 * (N / E)) void row_split_kernel(const Ins
     if (threadIdx.x == 0) run.form = FORM_HYBRID;
   }
   // Real-space normalization from the column pass's k-space sums (Parseval).
-  const double nrm = wave_sum_strided(P.part + PART_NRM * nt2, nt2);
+  const double nrm = psum.sum();
   const C* tw = stw.store(reinterpret_cast<C*>(smem) + ROWS * 2 * N);
   if constexpr (kTw) __syncthreads();  // publishes the twiddles to every wave
   const double lam2 = P.atom_num / (P.dv_r * (double)N * (double)ny * nrm);

@@ -192,7 +192,7 @@ __global__ __launch_bounds__(RROWS*(N / RE)) void persist_steps_kernel(PersistAr
         const InstDev& P = a.insts[inst];
         C* psi = reinterpret_cast<C*>(a.direct_psi ? a.direct_psi : P.psi);
         const RunDev& run = a.runs[inst];
-        row_item<R, N, RE, RROWS, false, CM>(P, psi, N, twx, dur, CW, a.row_stream, blk, smem, [&]() -> bool {
+        row_item<R, N, RE, RROWS, false, CM>(P, psi, N, P.part, twx, dur, CW, a.row_stream, blk, smem, [&]() -> bool {
           // The first sub-step of a full step records the previous step's
           // populations (row block 0 of the slot).
           if (j == 0 && blk == 0) record_pops<(CM & CM_LOAD) != 0>(P, run.pops, run.pops_cap, s_step0[li] + k, kColPer);

@@ -12,10 +12,11 @@ namespace sgpe {
 // Split-step pass launchers; with non-null events the launch carries them
 // (hipExtLaunchKernelGGL), which timestamps the kernel's own execution.
 // The void*/int pair is the direct state address and length (null: read
-// from the slot table).
+// from the slot table); rows take the direct partial sums' address as well.
 typedef void (*ColFn)(dim3, dim3, size_t, hipStream_t, hipEvent_t, hipEvent_t, const InstDev*, RunDev*, void*, int,
                       const void*, int, int, int, int);
-typedef void (*RowFn)(dim3, dim3, size_t, hipStream_t, hipEvent_t, hipEvent_t, const InstDev*, RunDev*, void*, int,
+typedef void (*RowFn)(dim3, dim3, size_t, hipStream_t, hipEvent_t, hipEvent_t, const InstDev*, RunDev*, void*,
+                      const double*, int,
                       const void*, int, int, int, int);
 typedef void (*FRowFn)(dim3, dim3, size_t, hipStream_t, FftPair, int, int, double, const void*);
 typedef void (*FColFn)(dim3, dim3, size_t, hipStream_t, FftPair, int, int, const void*);
@@ -52,24 +53,36 @@ void col_launch(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent
 }
 template <typename R, int N, int E, int ROWS, bool G>
 void row_launch(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const InstDev* i, RunDev* r,
-                void* dpsi, int dn, const void* tw, int dur, int first, int colw, int st) {
+                void* dpsi, const double* dpart, int dn, const void* tw, int dur, int first, int colw, int st) {
   typedef typename Cx<R>::T C;
+  if constexpr (row_has_held<R, N, E>()) {
+    if ((size_t)g.x * g.z <= (size_t)kCus && !e0) {
+      hipLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G, true>), g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur,
+                         first, colw, st);
+      return;
+    }
+    if ((size_t)g.x * g.z <= (size_t)kCus) {
+      hipExtLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G, true>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi,
+                            dpart, dn, (const C*)tw, dur, first, colw, st);
+      return;
+    }
+  }
   if (e0)
-    hipExtLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi, dn,
+    hipExtLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi, dpart, dn,
                           (const C*)tw, dur, first, colw, st);
   else
-    hipLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G>), g, b, l, s, i, r, dpsi, dn, (const C*)tw, dur, first, colw,
+    hipLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G>), g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur, first, colw,
                        st);
 }
 template <typename R, int N, int E, int ROWS, bool G>
 void rowsplit_launch(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const InstDev* i,
-                     RunDev* r, void* dpsi, int dn, const void* tw, int dur, int first, int colw, int st) {
+                     RunDev* r, void* dpsi, const double* dpart, int dn, const void* tw, int dur, int first, int colw, int st) {
   typedef typename Cx<R>::T C;
   if (e0)
-    hipExtLaunchKernelGGL((row_split_kernel<R, N, E, ROWS, G>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi, dn,
+    hipExtLaunchKernelGGL((row_split_kernel<R, N, E, ROWS, G>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi, dpart, dn,
                           (const C*)tw, dur, first, colw, st);
   else
-    hipLaunchKernelGGL((row_split_kernel<R, N, E, ROWS, G>), g, b, l, s, i, r, dpsi, dn, (const C*)tw, dur, first,
+    hipLaunchKernelGGL((row_split_kernel<R, N, E, ROWS, G>), g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur, first,
                        colw, st);
 }
 template <typename R, int N, int E, int ROWS>
