@@ -141,6 +141,29 @@ static void default_col(int prec, int n, int* e, int* w) {
   }
 }
 
+// Row-pass shape of a new plan (before any tuning): short rows of few
+// instances take small radices and tiles, which spread them over more
+// workgroups and shorten each one's chain. `rows` = grid rows x slots.
+// Dispatch times with the default tile above and with these: 64 points, 64
+// rows 6.1 -> 4.3 us (complex128, imaginary time), 128 points, 64 rows 7.1 -> 4.6,
+// 256 points, 64 rows 7.5 -> 5.0; up to 4096 rows 64 points 9.6 -> 8.7; from
+// there on the default tile is the faster one (128 points, 8192 rows 17.5
+// against 20).
+static void default_row_pass(int prec, int n, long rows, int* e, int* r) {
+  default_row(prec, n, e, r);
+  if (rows <= 1024) {
+    switch (n) {
+      case 64: *e = 2; *r = 2; break;
+      case 128: *e = 2; *r = 1; break;
+      case 256: *e = 4; *r = -1; break;
+      default: break;
+    }
+  } else if (rows <= 4096 && n <= 128) {
+    *e = 4;
+    *r = 4;
+  }
+}
+
 static int set_lds_attr(const void* kernel, size_t bytes) {
   if (bytes > 64 * 1024) HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
   return SGPE_OK;
@@ -1548,7 +1571,7 @@ int sgpe_plan_create(sgpe_ctx* ctx, int precision, int ny, int nx, int n_slots, 
     // Compiled default shapes where they fit the grid, else the runtime-length
     // kernels for that axis (e = 0).
     int re, rr, ce, cw;
-    default_row(precision, nx, &re, &rr);
+    default_row_pass(precision, nx, (long)ny * n_slots, &re, &rr);
     default_col(precision, ny, &ce, &cw);
     if (!fit_shape(K_ROW, precision, nx, ny, &re, &rr)) re = 0;
     if (!fit_shape(K_COL, precision, ny, nx, &ce, &cw)) ce = 0;
