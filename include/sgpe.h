@@ -130,6 +130,15 @@ int sgpe_norm(sgpe_ctx* ctx, int precision, int ny, int nx, void* psi0, void* ps
 int sgpe_norm_noalloc(sgpe_ctx* ctx, int precision, int ny, int nx, void* psi0, void* psi1, double vol_elem,
                       double atom_num, void* dens0, void* dens1, double* nf_out);
 
+/* norm out of place: in0, in1 are left as they are, out0, out1 (not
+ * overlapping them, or equal to them) receive the normalized components, dens0
+ * and dens1 (optional) the densities. The reduction's partials go to the
+ * caller's device memory `scratch` (count doubles; SGPE_NORM_SCRATCH fit any
+ * grid), so calls on different streams do not share any. Asynchronous. */
+#define SGPE_NORM_SCRATCH 2049
+int sgpe_norm_into(sgpe_ctx* ctx, int precision, int ny, int nx, const void* in0, const void* in1, double vol_elem,
+                   double atom_num, void* out0, void* out1, void* dens0, void* dens1, double* scratch, int count);
+
 /* calc_pops (tensor_tools.py:466-484): out2[s] = vol_elem * sum |psi_s|^2,
  * written to HOST memory (synchronizes the stream). */
 int sgpe_pops(sgpe_ctx* ctx, int precision, int ny, int nx, const void* psi0, const void* psi1, double vol_elem,

@@ -350,6 +350,7 @@ static const PEntry* find_persist(int prec, int n, int re, int rr, int ce, int c
 // each device (scratch_addr).
 static constexpr int kNormBlocks = 1024;
 static constexpr int kNormScratchDoubles = 2 * kNormBlocks + 32;
+static_assert(SGPE_NORM_SCRATCH >= 2 * kNormBlocks + 1, "norm partials of any grid and the norm factor");
 static __device__ __align__(256) double scratch[kNormScratchDoubles];
 
 // Device address of `scratch` on `device`, looked up once per device (with
@@ -1465,24 +1466,28 @@ int sgpe_fft2(sgpe_ctx* ctx, int precision, int ny, int nx, int n_arrays, void* 
 
 static int reduce_blocks(size_t n) { return (int)std::min<size_t>((n + 255) / 256, kNormBlocks); }
 
-// norm() on the context's stream with the partials and norm factor in
-// `part` (2 nb + 1 doubles, nb = reduce_blocks(ny nx)).
-static int launch_norm(sgpe_ctx* ctx, int precision, int ny, int nx, void* psi0, void* psi1, double vol_elem,
-                       double atom_num, void* dens0, void* dens1, double* nf_out, double* part) {
+// norm() of in0, in1 into out0, out1 (which may be the same arrays) on the
+// context's stream with the partials and norm factor in `part` (2 nb + 1
+// doubles, nb = reduce_blocks(ny nx)).
+static int launch_norm(sgpe_ctx* ctx, int precision, int ny, int nx, const void* in0, const void* in1, double vol_elem,
+                       double atom_num, void* out0, void* out1, void* dens0, void* dens1, double* nf_out,
+                       double* part) {
   const size_t n = (size_t)ny * nx;
   const int nb = reduce_blocks(n);
   double* nf_dev = part + 2 * nb;
   if (precision == SGPE_C128) {
-    hipLaunchKernelGGL(density_sums_kernel<double>, dim3(nb), dim3(256), 0, ctx->stream, (const double2*)psi0,
-                       (const double2*)psi1, n, part);
-    hipLaunchKernelGGL(norm_apply_kernel<double>, dim3(nb), dim3(256), 0, ctx->stream, (double2*)psi0,
-                       (double2*)psi1, n, (const double*)part, nb, vol_elem, atom_num, (double*)dens0,
+    hipLaunchKernelGGL(density_sums_kernel<double>, dim3(nb), dim3(256), 0, ctx->stream, (const double2*)in0,
+                       (const double2*)in1, n, part);
+    hipLaunchKernelGGL(norm_apply_kernel<double>, dim3(nb), dim3(256), 0, ctx->stream, (const double2*)in0,
+                       (const double2*)in1, n, (const double*)part, nb, vol_elem, atom_num, (double2*)out0,
+                       (double2*)out1, (double*)dens0,
                        (double*)dens1, nf_dev);
   } else {
-    hipLaunchKernelGGL(density_sums_kernel<float>, dim3(nb), dim3(256), 0, ctx->stream, (const float2*)psi0,
-                       (const float2*)psi1, n, part);
-    hipLaunchKernelGGL(norm_apply_kernel<float>, dim3(nb), dim3(256), 0, ctx->stream, (float2*)psi0,
-                       (float2*)psi1, n, (const double*)part, nb, vol_elem, atom_num, (float*)dens0,
+    hipLaunchKernelGGL(density_sums_kernel<float>, dim3(nb), dim3(256), 0, ctx->stream, (const float2*)in0,
+                       (const float2*)in1, n, part);
+    hipLaunchKernelGGL(norm_apply_kernel<float>, dim3(nb), dim3(256), 0, ctx->stream, (const float2*)in0,
+                       (const float2*)in1, n, (const double*)part, nb, vol_elem, atom_num, (float2*)out0,
+                       (float2*)out1, (float*)dens0,
                        (float*)dens1, nf_dev);
   }
   HIP_TRY(hipGetLastError());
@@ -1503,7 +1508,8 @@ int sgpe_norm(sgpe_ctx* ctx, int precision, int ny, int nx, void* psi0, void* ps
     const int nb = reduce_blocks((size_t)ny * nx);
     int rc = ctx_reduction(ctx, 2 * (size_t)nb + 1);
     if (rc) return rc;
-    return launch_norm(ctx, precision, ny, nx, psi0, psi1, vol_elem, atom_num, dens0, dens1, nf_out, ctx->red);
+    return launch_norm(ctx, precision, ny, nx, psi0, psi1, vol_elem, atom_num, psi0, psi1, dens0, dens1, nf_out,
+                       ctx->red);
   });
 }
 
@@ -1517,8 +1523,20 @@ int sgpe_norm_noalloc(sgpe_ctx* ctx, int precision, int ny, int nx, void* psi0, 
       return fail(SGPE_E_ARG, "sgpe_norm_noalloc: the reduction needs more than the 16.6 KiB scratch");
     if (!ctx->scratch_dev) return fail(SGPE_E_HIP, "sgpe_norm_noalloc: no scratch address for this device");
     HIP_TRY(hipSetDevice(ctx->device));
-    return launch_norm(ctx, precision, ny, nx, psi0, psi1, vol_elem, atom_num, dens0, dens1, nf_out,
+    return launch_norm(ctx, precision, ny, nx, psi0, psi1, vol_elem, atom_num, psi0, psi1, dens0, dens1, nf_out,
                        ctx->scratch_dev);
+  });
+}
+
+int sgpe_norm_into(sgpe_ctx* ctx, int precision, int ny, int nx, const void* in0, const void* in1, double vol_elem,
+                   double atom_num, void* out0, void* out1, void* dens0, void* dens1, double* scratch, int count) {
+  return guarded([&]() -> int {
+    if (!ctx || !in0 || !in1 || !out0 || !out1 || !scratch || ny <= 0 || nx <= 0) return fail(SGPE_E_ARG, "bad arguments");
+    if (precision != SGPE_C128 && precision != SGPE_C64) return fail(SGPE_E_ARG, "bad precision");
+    const int nb = reduce_blocks((size_t)ny * nx);
+    if (count < 2 * nb + 1) return fail(SGPE_E_ARG, "scratch is too small (SGPE_NORM_SCRATCH doubles fit any grid)");
+    HIP_TRY(hipSetDevice(ctx->device));
+    return launch_norm(ctx, precision, ny, nx, in0, in1, vol_elem, atom_num, out0, out1, dens0, dens1, nullptr, scratch);
   });
 }
 

@@ -69,6 +69,7 @@ def _declare(lib):
         'sgpe_fft2': (i, [vp, i, i, i, i, ctypes.POINTER(vp), ctypes.POINTER(vp), i, d, d]),
         'sgpe_norm': (i, [vp, i, i, i, vp, vp, d, d, vp, vp, _dp]),
         'sgpe_norm_noalloc': (i, [vp, i, i, i, vp, vp, d, d, vp, vp, _dp]),
+        'sgpe_norm_into': (i, [vp, i, i, i, vp, vp, d, d, vp, vp, vp, vp, vp, i]),
         'sgpe_pops': (i, [vp, i, i, i, vp, vp, d, _dp]),
         'sgpe_plan_create': (i, [vp, i, i, i, i, ctypes.POINTER(vp)]),
         'sgpe_plan_destroy': (None, [vp]),
@@ -219,14 +220,31 @@ def fft2(arrays, inverse, dx, dy, out=None):
     return outs
 
 
+NORM_SCRATCH = 2049  # SGPE_NORM_SCRATCH
+
+
 def norm(psi, vol_elem, atom_num):
-    """Device norm(): returns (normalized psi list, density list)."""
-    p0, p1 = (p.clone() for p in psi)
+    """Device norm(): returns (normalized psi list, density list).
+
+    Contiguous pairs of one kind go out of place without a copy first and
+    without waiting for the stream; the partials' scratch comes from torch's
+    allocator, so calls on different streams share none. Other pairs are
+    copied and normalized in place."""
+    a, b = psi
+    plain = (a.shape == b.shape and a.dtype == b.dtype and a.device == b.device and a.is_contiguous()
+             and b.is_contiguous() and not (a.requires_grad or b.requires_grad or a.is_conj() or b.is_conj()
+                      or a.is_neg() or b.is_neg()))
+    p0, p1 = (torch.empty_like(a), torch.empty_like(b)) if plain else (a.clone(), b.clone())
     prec = precision_of(p0.dtype)
     ny, nx = p0.shape
     d0 = torch.empty((ny, nx), dtype=REAL_DTYPE[prec], device=p0.device)
     d1 = torch.empty_like(d0)
     ctx = Context.get(p0.device)
+    if plain:
+        scratch = torch.empty(NORM_SCRATCH, dtype=torch.float64, device=p0.device)
+        check(lib().sgpe_norm_into(ctx.handle, prec, ny, nx, _ptr(a), _ptr(b), float(vol_elem), float(atom_num),
+                                   _ptr(p0), _ptr(p1), _ptr(d0), _ptr(d1), _ptr(scratch), NORM_SCRATCH))
+        return [p0, p1], [d0, d1]
     nf = ctypes.c_double()
     check(lib().sgpe_norm(ctx.handle, prec, ny, nx, _ptr(p0), _ptr(p1), float(vol_elem),
                           float(atom_num), _ptr(d0), _ptr(d1), ctypes.byref(nf)))
