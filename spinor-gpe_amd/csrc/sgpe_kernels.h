@@ -1082,10 +1082,9 @@ template <typename R, int N, int E, int ROWS> constexpr int row_min_waves() {
 }
 
 // HELD: for launches of at most one workgroup per CU, where registers limit
-// nothing: addresses and twiddles kept from the inverse
-// transform to the forward one (at the price of a few spills). Complex128
-// 2048-point rows, 256 of them: 21.3 us
-// instead of 24.7; with 2048 of them it would be 98 instead of 79.
+// nothing: addresses and twiddles kept from the inverse transform to the
+// forward one (at the price of a few spills). Complex128 2048-point rows, 256 of
+// them: 21.3 us instead of 24.7; with 2048 of them it would be 98 instead of 79.
 constexpr int kCus = 256;
 template <typename R, int N, int E> constexpr bool row_has_held() { return sizeof(R) == 8 && N == 2048 && E == 8; }
 template <typename R, int N, int E, int ROWS, bool GENERAL, bool HELD = false>
@@ -1099,9 +1098,10 @@ __global__ __launch_bounds__(ROWS*(N / E), (row_min_waves<R, N, E, ROWS>())) voi
   const int inst = blockIdx.z;
   RunDev& run = runs[inst];
   const InstDev& P = insts[inst];
-  // State and partial sums' addresses and column length: kernel arguments for a single-slot
-  // plan (loads first, active flag checked after them), else read together
-  // with the active flag (one round of scalar loads before the state loads).
+  // Addresses of the state and the partial sums, and the column length: kernel
+  // arguments for a single-slot plan (loads first, active flag checked after
+  // them), else read together with the active flag (one round of scalar loads
+  // before the state loads).
   const bool direct = direct_psi != nullptr;
   C* const psi = reinterpret_cast<C*>(direct ? direct_psi : P.psi);
   const int ny = direct ? direct_n : P.ny;

@@ -4,7 +4,7 @@
 //
 // A length is split on the host into two to five radices of at most 16
 // (mix_factor). A stage is one register butterfly of compile-time radix per
-// work item (a uniform switch picks the radix), data pass between stages through
+// work item (a uniform switch picks the radix); data pass between stages through
 // LDS. A pass runs
 //     stage 0 (global -> LDS), inner stages (LDS -> LDS), last stage,
 //     pointwise block, then the adjoint stages back in reverse order:
@@ -14,8 +14,8 @@
 // LDS; the column pass applies its factors between the two in registers), and
 // its last stage writes to global memory what stage 0 read. Against keeping the
 // data in LDS throughout, with one stage per prime power, twiddles gathered from
-// global memory and two LDS buffers (sgpe_generic.h), a 600-point pass makes 4
-// round trips through LDS instead of 10.
+// global memory and two LDS buffers (sgpe_generic.h), a 600-point column
+// pass makes 4 round trips through LDS instead of 10 (the row pass 6).
 //
 // Bound by latency on grids of this size (one or two workgroups per CU: each
 // stage is an LDS round trip and a barrier), by LDS and vector instructions in
@@ -39,7 +39,7 @@ constexpr int kMixThreads = 512;  // most threads of a workgroup
 
 // One stage: radix, span (product of the radices before it), butterflies,
 // offset of its twiddles, and multipliers for exact division of 16-bit numbers
-// by span and butterflies (ceil(2^32 / d)).
+// by span and butterflies (floor(2^32 / d) + 1).
 struct MixStage {
   int radix, span, nb, off;
   unsigned div_span, div_nb;
