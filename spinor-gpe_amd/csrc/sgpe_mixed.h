@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "sgpe_kernels.h"
+#include "sgpe_units.h"
 
 namespace sgpe {
 
@@ -56,35 +57,6 @@ __device__ __forceinline__ int mix_div(int x, int d, unsigned m) {
 }
 
 // ------------------------------------------------------ register butterflies
-
-// cos and sin of 2 pi m / R at compile time, the angle reduced to [0, pi/4].
-constexpr double mix_series(double x, bool cosine) {
-  double term = cosine ? 1.0 : x, sum = 0.0;
-  for (int i = cosine ? 1 : 2; i < 30; i += 2) {
-    sum += term;
-    term *= -x * x / (i * (i + 1));
-  }
-  return sum;
-}
-constexpr double mix_cos(int m, int r) {
-  m = ((m % r) + r) % r;
-  if (2 * m > r) m = r - m;                                  // [0, pi]
-  if (4 * m > r) return -mix_cos(r - 2 * m, 2 * r);          // pi - angle
-  if (8 * m > r) return mix_series(1.57079632679489661923 * (r - 4 * m) / r, false);  // sin(pi/2 - angle)
-  return mix_series(6.28318530717958647692 * m / r, true);
-}
-constexpr double mix_sin(int m, int r) { return mix_cos(4 * m - r, 4 * r); }
-
-template <int R> struct MixUnit {
-  double c[R], s[R];
-  constexpr MixUnit() : c{}, s{} {
-    for (int m = 0; m < R; ++m) {
-      c[m] = mix_cos(m, R);
-      s[m] = mix_sin(m, R);
-    }
-  }
-};
-template <int R> struct MixUnitTable { static constexpr MixUnit<R> u{}; };
 
 // Odd prime radix: sums and differences of opposite inputs. From radix 7 on the
 // products and sums run in double also for complex64 (the same instruction
