@@ -142,25 +142,25 @@ static void default_col(int prec, int n, int* e, int* w) {
 }
 
 // Row-pass shape of a new plan (before any tuning): short rows of few
-// instances take small radices and tiles, which spread them over more
-// workgroups and shorten each one's chain. `rows` = grid rows x slots.
-// Dispatch times with the default tile above and with these: 64 points, 64
-// rows 6.1 -> 4.3 us (complex128, imaginary time), 128 points, 64 rows 7.1 -> 4.6,
-// 256 points, 64 rows 7.5 -> 5.0; up to 4096 rows 64 points 9.6 -> 8.7; from
-// there on the default tile is the faster one (128 points, 8192 rows 17.5
-// against 20).
+// instances take small tiles, which spread them over more workgroups and
+// shorten each one's chain. `rows` = grid rows x slots. Radix 4, not 2: two
+// butterfly levels between twiddles leave a radix-4 pass as exact as the default
+// radix 8 (complex64 ground-state steps of 64^2: 6.4e-7 and 6.2e-7 from 64
+// bits, radix 2 7.8e-7; 128^2: 5.9e-7, 6.1e-7 and 7.6e-7). Dispatch times in
+// imaginary time, complex128 (complex64), us, with the default tile above ->
+// here -> radix 2: 64 points, 64 rows 6.05 -> 4.37 -> 4.23 (4.60 -> 4.23 -> 4.22), 1024
+// rows 6.51 -> 4.92 -> 4.98, 4096 rows 9.67 -> 8.84 -> 9.73; 128 points, 64 rows 6.56 ->
+// 5.36 -> 4.93 (6.13 -> 4.52 -> 4.26), 4096 rows 15.7 -> 14.3; 256 points, 64 rows
+// 6.96 -> 4.41. From 8192 rows on the default tile is the faster one for 128
+// points (18.9 against 20.3), from 4096 rows of 256 points on equal (16.4, 17.5).
 static void default_row_pass(int prec, int n, long rows, int* e, int* r) {
   default_row(prec, n, e, r);
-  if (rows <= 1024) {
-    switch (n) {
-      case 64: *e = 2; *r = 2; break;
-      case 128: *e = 2; *r = 1; break;
-      case 256: *e = 4; *r = -1; break;
-      default: break;
-    }
-  } else if (rows <= 4096 && n <= 128) {
+  if (rows <= 4096 && n <= 128) {
     *e = 4;
-    *r = 4;
+    *r = n == 128 && rows <= 1024 ? 2 : 4;
+  } else if (rows <= 1024 && n == 256) {
+    *e = 4;
+    *r = -1;
   }
 }
 

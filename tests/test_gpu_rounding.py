@@ -5,7 +5,9 @@ error of the shape in question against that of radix 8 on the same grid.
 
 Radix-16 columns: the rounded cos(pi/8) alone is the same in every butterfly
 and made the error 1.09 (256 points) and 1.16 times (1024) that of radix 8, with
-its low part 0.92 and 0.85. Bound 1.1."""
+its low part 0.92 and 0.85. Default rows of new plans: radix 2 on short rows
+rounds at a twiddle per level, 1.11 (64 points) and 1.15 times (128); radix 4
+1.00. Bound 1.1."""
 
 import itertools
 
@@ -49,3 +51,12 @@ def test_radix_16_columns(gpu, n):
     e16, e8 = (_error(gpu, n, n, row, col) for col in ((16, 8), (8, 4)))
     print(f"[rounding] columns {n}: radix 16 {e16:.3e}, radix 8 {e8:.3e}", flush=True)
     assert e16 < 1.1 * e8, (e16, e8)
+
+
+@pytest.mark.parametrize('n', [64, 128])
+def test_default_rows(gpu, monkeypatch, tmp_path, n):
+    """96 rows: no entry of the shape table, so the default shape by the number of rows."""
+    monkeypatch.setenv('SGPE_TUNE_FILE', str(tmp_path / 'none.json'))
+    default, e8 = (_error(gpu, n, 96, row) for row in (None, (8, 8 if n == 64 else 4)))
+    print(f"[rounding] rows {n}: default {default:.3e}, radix 8 {e8:.3e}", flush=True)
+    assert default < 1.1 * e8, (default, e8)
