@@ -379,7 +379,9 @@ struct sgpe_ctx {
   int n_cu = 0;                      // compute units (residency check of persistent launches)
   hipStream_t stream = nullptr;
   hipStream_t cap_stream = nullptr;  // private stream used only for graph capture
+  std::mutex mu;                     // guards tw and mix: calls of several threads share a context
   std::map<int, void*> tw;           // stage-major twiddles, key (prec*8192 + n)*32 + e
+  std::map<int, MixFft> mix;         // mix_factor of the lengths asked for so far
   double* red = nullptr;             // reduction scratch for primitives
   size_t red_count = 0;
   double* red_host = nullptr;        // pinned
@@ -391,6 +393,7 @@ struct sgpe_ctx {
 // w_{L R}^{r k} (k < L, 1 <= r < R) at (L - 1) + k (R - 1) + (r - 1).
 static int ctx_twiddles(sgpe_ctx* ctx, int prec, int n, int e, const void** out) {
   const int key = (prec * 8192 + n) * 32 + e;
+  std::lock_guard<std::mutex> lock(ctx->mu);
   auto it = ctx->tw.find(key);
   if (it != ctx->tw.end()) {
     *out = it->second;
@@ -461,6 +464,7 @@ static void root_of_unity(int m, int n, double* re, double* im) {
 
 // Device table of n complex entries value(i, &re, &im), cached under `key`.
 template <class F> static int ctx_table(sgpe_ctx* ctx, int key, int prec, int n, F value, const void** out) {
+  std::lock_guard<std::mutex> lock(ctx->mu);
   auto it = ctx->tw.find(key);
   if (it != ctx->tw.end()) {
     *out = it->second;
@@ -494,20 +498,27 @@ static int ctx_roots(sgpe_ctx* ctx, int prec, int n, const void** out) {
   return ctx_table(ctx, key, prec, n, [n](int m, double* re, double* im) { root_of_unity(m, n, re, im); }, out);
 }
 
+// mix_factor(n), searched for once per length: the search takes up to 2 us, a
+// sixth of a small transform's call.
+static const MixFft& ctx_mix(sgpe_ctx* ctx, int n) {
+  std::lock_guard<std::mutex> lock(ctx->mu);
+  auto it = ctx->mix.find(n);
+  if (it == ctx->mix.end()) it = ctx->mix.emplace(n, mix_factor(n)).first;
+  return it->second;
+}
+
 // Stage-major twiddles of the mixed-radix kernels: the stage of span L and
 // radix R keeps w_{L R}^{r k} (k < L, 1 <= r < R) at (L - 1) + k (R - 1) +
-// (r - 1).
+// (r - 1). The last entry is not read.
 static int ctx_mix_twiddles(sgpe_ctx* ctx, int prec, const MixFft& f, const void** out) {
   const int n = f.n;
   const int key = (prec * 8192 + n) * 32 + 17;  // compiled shapes: e <= 16
-  std::vector<int> power(n, 0);  // entry i is exp(-2 pi i power[i] / n)
-  for (int s = 0; s < f.ns; ++s) {
-    const int L = f.st[s].span, R = f.st[s].radix;
-    for (int k = 0; k < L; ++k)
-      for (int r = 1; r < R; ++r) power[f.st[s].off + k * (R - 1) + r - 1] = r * k * (n / (L * R));
-  }
-  return ctx_table(ctx, key, prec, n,
-                   [&](int i, double* re, double* im) { root_of_unity(power[i], n, re, im); }, out);
+  return ctx_table(ctx, key, prec, n, [&f, n](int i, double* re, double* im) {
+    int s = f.ns - 1;
+    while (f.st[s].off > i) --s;
+    const int L = f.st[s].span, R = f.st[s].radix, j = i - f.st[s].off;
+    root_of_unity((j / (R - 1)) * (j % (R - 1) + 1) * (n / (L * R)), n, re, im);
+  }, out);
 }
 
 // Dynamic LDS of a kernel with data_bytes of exchange buffers for n-point
@@ -639,13 +650,13 @@ static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col
   MixFft mx{}, my{};
   int mrows = 0, mw = 0;
   if (gx) {
-    mx = mix_factor(p->nx);
+    mx = ctx_mix(p->ctx, p->nx);
     if (mx.ns) mrows = mix_batch(mx, p->ny, p->nslots, cs, 1, 4, 2, 2L * std::max(p->ctx->n_cu, 1));
     if (!mrows) mx.ns = 0;
     row_rows = 1;
   }
   if (gy) {
-    my = mix_factor(p->ny);
+    my = ctx_mix(p->ctx, p->ny);
     if (my.ns)
       mw = mix_batch(my, p->nx, 2L * p->nslots, cs, (int)(64 / cs), (int)(128 / cs), 1, 2L * std::max(p->ctx->n_cu, 1));
     if (!mw) my.ns = 0;
@@ -1362,12 +1373,12 @@ int sgpe_fft2(sgpe_ctx* ctx, int precision, int ny, int nx, int n_arrays, void* 
     int mrows = 0, mw = 0;
     const long per_launch = std::min(n_arrays, 2), want = 2L * std::max(ctx->n_cu, 1);
     if (gx) {
-      mx = mix_factor(nx);
+      mx = ctx_mix(ctx, nx);
       if (mx.ns) mrows = mix_batch(mx, ny, per_launch, cs, 1, 8, 1, want);
       if (!mrows) mx.ns = 0;
     }
     if (gy) {
-      my = mix_factor(ny);
+      my = ctx_mix(ctx, ny);
       if (my.ns) mw = mix_batch(my, nx, per_launch, cs, (int)(64 / cs), (int)(128 / cs), 1, want);
       if (!mw) my.ns = 0;
     }
