@@ -691,6 +691,8 @@ static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col
   } else {
     rc = set_lds_attr(r->kernel, rl);
     if (!rc) rc = set_lds_attr(r->kernel_g, rl);
+    for (const void* k : r->held)
+      if (!rc && k) rc = set_lds_attr(k, rl);
     if (!rc) rc = ctx_twiddles(p->ctx, p->prec, p->nx, row_e, &twx);
   }
   if (rc) return rc;
@@ -816,10 +818,10 @@ static void launch_row(sgpe_plan* p, hipStream_t s, int dur, int first, hipEvent
   }
   const size_t lds = row_pass_lds(p->row_e, p->row_rows, p->nx, csize(p->prec));
   dim3 grid(p->ny / std::abs(p->row_rows), 1, p->nlaunch), block(row_block_threads(p->row_e, p->row_rows, p->nx));
+  const bool held = p->row->held[0] && (long)grid.x * grid.z <= p->ctx->n_cu;
   ((RowFn)(p->general_row ? p->row->launch_g : p->row->launch))(grid, block, lds, s, e0, e1, p->d_inst, p->d_run,
                                                                 direct_state(p), p->h_inst[0].part, p->ny, p->tw_x, dur,
-                                                                first, p->col_w,
-                                                                p->row_stream);
+                                                                first, p->col_w, p->row_stream, held);
 }
 
 static void issue_sub_step(sgpe_plan* p, hipStream_t s, int which, int first) {

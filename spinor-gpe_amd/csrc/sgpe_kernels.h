@@ -1081,11 +1081,11 @@ template <typename R, int N, int E, int ROWS> constexpr int row_min_waves() {
   return E >= 8 && cs == 16 && waves >= 2 ? 2 : 1;
 }
 
-// HELD: for launches of at most one workgroup per CU, where registers limit
-// nothing: addresses and twiddles kept from the inverse transform to the
-// forward one (at the price of a few spills). Complex128 2048-point rows, 256 of
-// them: 21.3 us instead of 24.7; with 2048 of them it would be 98 instead of 79.
-constexpr int kCus = 256;
+// HELD: for launches of at most one workgroup per CU (launch_row), where
+// registers limit nothing: addresses and twiddles kept from the inverse
+// transform to the forward one (at the price of a few spills). Complex128
+// 2048-point rows, 256 of them: 21.3 us instead of 24.7; with 2048 of them it
+// would be 98 instead of 79.
 template <typename R, int N, int E> constexpr bool row_has_held() { return sizeof(R) == 8 && N == 2048 && E == 8; }
 template <typename R, int N, int E, int ROWS, bool GENERAL, bool HELD = false>
 __global__ __launch_bounds__(ROWS*(N / E), (row_min_waves<R, N, E, ROWS>())) void row_pass_kernel(const InstDev* __restrict__ insts,

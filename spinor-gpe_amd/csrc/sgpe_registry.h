@@ -12,12 +12,12 @@ namespace sgpe {
 // Split-step pass launchers; with non-null events the launch carries them
 // (hipExtLaunchKernelGGL), which timestamps the kernel's own execution.
 // The void*/int pair is the direct state address and length (null: read
-// from the slot table); rows take the direct partial sums' address as well.
+// from the slot table); rows take the direct partial sums' address as well,
+// and whether to run the HELD variant (row_pass_kernel) of shapes that have one.
 typedef void (*ColFn)(dim3, dim3, size_t, hipStream_t, hipEvent_t, hipEvent_t, const InstDev*, RunDev*, void*, int,
                       const void*, int, int, int, int);
 typedef void (*RowFn)(dim3, dim3, size_t, hipStream_t, hipEvent_t, hipEvent_t, const InstDev*, RunDev*, void*,
-                      const double*, int,
-                      const void*, int, int, int, int);
+                      const double*, int, const void*, int, int, int, int, int);
 typedef void (*FRowFn)(dim3, dim3, size_t, hipStream_t, FftPair, int, int, double, const void*);
 typedef void (*FColFn)(dim3, dim3, size_t, hipStream_t, FftPair, int, int, const void*);
 typedef void (*EFn)(dim3, dim3, size_t, hipStream_t, const InstDev*, const RunDev*, const void*);
@@ -28,6 +28,7 @@ struct KEntry {
   const void* kernel;
   void* launch_g;  // split-step passes: the variant for dense operators
   const void* kernel_g;
+  const void* held[2];  // row shapes with a HELD variant: its two kernels, else null
 };
 
 struct KTable {
@@ -51,39 +52,40 @@ void col_launch(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent
     hipLaunchKernelGGL((col_pass_kernel<R, N, E, W, G, GKY>), g, b, l, s, i, r, dpsi, dn, (const C*)tw, m, dp, dc,
                        st);
 }
+template <typename R, int N, int E, int ROWS, bool G> constexpr const void* held_kernel() {
+  if constexpr (row_has_held<R, N, E>())
+    return (const void*)&row_pass_kernel<R, N, E, ROWS, G, true>;
+  else
+    return nullptr;
+}
 template <typename R, int N, int E, int ROWS, bool G>
 void row_launch(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const InstDev* i, RunDev* r,
-                void* dpsi, const double* dpart, int dn, const void* tw, int dur, int first, int colw, int st) {
+                void* dpsi, const double* dpart, int dn, const void* tw, int dur, int first, int colw, int st,
+                int held) {
   typedef typename Cx<R>::T C;
+  auto launch = [&](auto kernel) {
+    if (e0)
+      hipExtLaunchKernelGGL(kernel, g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi, dpart, dn, (const C*)tw, dur, first,
+                            colw, st);
+    else
+      hipLaunchKernelGGL(kernel, g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur, first, colw, st);
+  };
   if constexpr (row_has_held<R, N, E>()) {
-    if ((size_t)g.x * g.z <= (size_t)kCus && !e0) {
-      hipLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G, true>), g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur,
-                         first, colw, st);
-      return;
-    }
-    if ((size_t)g.x * g.z <= (size_t)kCus) {
-      hipExtLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G, true>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi,
-                            dpart, dn, (const C*)tw, dur, first, colw, st);
-      return;
-    }
+    if (held) return launch(row_pass_kernel<R, N, E, ROWS, G, true>);
   }
-  if (e0)
-    hipExtLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi, dpart, dn,
-                          (const C*)tw, dur, first, colw, st);
-  else
-    hipLaunchKernelGGL((row_pass_kernel<R, N, E, ROWS, G>), g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur, first, colw,
-                       st);
+  launch(row_pass_kernel<R, N, E, ROWS, G>);
 }
 template <typename R, int N, int E, int ROWS, bool G>
 void rowsplit_launch(dim3 g, dim3 b, size_t l, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const InstDev* i,
-                     RunDev* r, void* dpsi, const double* dpart, int dn, const void* tw, int dur, int first, int colw, int st) {
+                     RunDev* r, void* dpsi, const double* dpart, int dn, const void* tw, int dur, int first, int colw,
+                     int st, int) {
   typedef typename Cx<R>::T C;
   if (e0)
     hipExtLaunchKernelGGL((row_split_kernel<R, N, E, ROWS, G>), g, b, (uint32_t)l, s, e0, e1, 0, i, r, dpsi, dpart, dn,
                           (const C*)tw, dur, first, colw, st);
   else
-    hipLaunchKernelGGL((row_split_kernel<R, N, E, ROWS, G>), g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur, first,
-                       colw, st);
+    hipLaunchKernelGGL((row_split_kernel<R, N, E, ROWS, G>), g, b, l, s, i, r, dpsi, dpart, dn, (const C*)tw, dur,
+                       first, colw, st);
 }
 template <typename R, int N, int E, int ROWS>
 void frow_launch(dim3 g, dim3 b, size_t l, hipStream_t s, FftPair io, int inv, int shift, double scale,
@@ -124,7 +126,8 @@ void erow_launch(dim3 g, dim3 b, size_t l, hipStream_t s, const InstDev* i, cons
    (void*)&sgpe::row_launch<R, N, E, RW, false>,                                                     \
    (const void*)&sgpe::row_pass_kernel<R, N, E, RW, false>,                                          \
    (void*)&sgpe::row_launch<R, N, E, RW, true>,                                                      \
-   (const void*)&sgpe::row_pass_kernel<R, N, E, RW, true>},
+   (const void*)&sgpe::row_pass_kernel<R, N, E, RW, true>,                                           \
+   {sgpe::held_kernel<R, N, E, RW, false>(), sgpe::held_kernel<R, N, E, RW, true>()}},
 // Column variant with the y phase tables in global memory, listed with
 // columns per block -W.
 #define SGPE_COLG_E(R, PR, N, E, W)                                                                  \
