@@ -246,9 +246,11 @@ int sgpe_plan_check(sgpe_plan* plan);
  * is timestamped by a hipEvent pair; *ms = its duration. Synchronizes. */
 int sgpe_profile_persistent(sgpe_plan* plan, int n_steps, double* ms);
 
-/* Cache policy of the two passes' state reads and writes: 1 = non-temporal
+/* Cache policy asked of the two passes' state reads and writes: 1 = non-temporal
  * (streaming) accesses, 0 = normal. Default: streaming for single-slot plans,
- * normal for batched ones. No reference counterpart (launch configuration). */
+ * normal for batched ones. Both run the same instructions in the present build
+ * (the compiler merges the two paths). No reference counterpart (launch
+ * configuration). */
 int sgpe_plan_set_streaming(sgpe_plan* plan, int row_stream, int col_stream);
 int sgpe_plan_get_streaming(const sgpe_plan* plan, int* out2);
 

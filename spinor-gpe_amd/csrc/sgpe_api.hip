@@ -236,10 +236,11 @@ static unsigned mix_magic(int d) { return (unsigned)((1ull << 32) / (unsigned)d 
 
 // Radices of an n-point transform: the fewest stages, then the smallest sum of
 // radices, then the smallest last radix from 4 on (of at most kMixMidRadix):
-// the last stage does both transforms' butterflies and the pointwise block, so
-// many items of few points there keep more threads busy. Stage 0, whose outputs go to LDS a
-// radix apart, takes the radix with the fewest factors of two (bank
-// conflicts). ns = 0: not a length of these kernels.
+// the last stage does both transforms' butterflies (the column pass with its
+// factors between them), so many items of few points there keep more threads
+// busy. Stage 0, whose outputs go to LDS a radix apart, takes the radix with the
+// fewest factors of two (bank conflicts). No length needs more than four stages.
+// ns = 0: not a length of these kernels.
 static MixFft mix_factor(int n) {
   MixFft f;
   std::memset(&f, 0, sizeof(f));

@@ -12,11 +12,12 @@
 // table of the length's roots of unity, root[m] = exp(-2 pi i m / n).
 // Radices above 7 take O(R) work per output: such lengths are supported,
 // not fast. Passes and transforms of 32 points and more without a prime factor
-// above 13 run the register kernels of sgpe_mixed.h instead; these here keep the
-// other lengths and every energy evaluation. The passes do what col_pass_kernel and
-// row_pass_kernel do (same sub-step schedule, same partial sums, same state
-// forms), so plans can mix them: a 96 x 128 grid takes the compiled
-// 128-point column pass and this row pass.
+// above 13 (twelve lengths from 1452 on apart) run the register kernels of
+// sgpe_mixed.h instead; these here keep the other lengths and every energy
+// evaluation. The passes do what col_pass_kernel and row_pass_kernel do (same
+// sub-step schedule, same partial sums, same state forms), so plans can mix
+// them: a 34 x 128 grid (nx = 34) takes the compiled 128-point column pass and
+// this row pass.
 #pragma once
 
 #include "sgpe_kernels.h"

@@ -29,9 +29,8 @@ namespace sgpe {
 // remainders): each fma(-k, Pi, r) rounds once, so r is within a few 1e-16
 // of x - k pi/2 for |k| < 1e15 (|x| < 1.5e15; beyond, a double no longer
 // resolves a radian of phase and the error grows with |x|). The quadrant is
-// k mod 4, computed exactly in double. Then Taylor polynomials in r (terms
-// through r^17 / r^18 for double, r^9 / r^10 for float: truncation below half
-// an ulp); within 2 ulp of the correctly rounded values. There is no
+// k mod 4, computed exactly in double. Then polynomials in r (sc_poly:
+// truncation below half an ulp); within 2 ulp of the correctly rounded values. There is no
 // library fallback: inlined at every call site, the device library's
 // large-argument code made the row pass's pointwise block twice as slow even
 // where it never ran (instruction fetch across it).
@@ -52,8 +51,8 @@ template <typename R> __device__ __forceinline__ void quadrant_fix(int q, R sr, 
 }
 
 // sin and cos for |r| <= pi/4. Double: minimax polynomials (Remez exchange,
-// relative error 3.4e-18 of sin, 5e-20 of cos before rounding; 2^-53-rounding
-// dominates: largest error 7.4e-17 and 9.6e-17, as the Taylor series with four
+// relative error with the rounded coefficients 5.9e-18 of sin, 1.2e-18 of cos;
+// 2^-53-rounding dominates: largest error 7.4e-17 and 9.6e-17, as the Taylor series with four
 // more terms has). Float: Taylor terms through r^9 / r^10.
 __device__ __forceinline__ void sc_poly(double r, double* s, double* c) {
   const double r2 = r * r;
@@ -104,8 +103,9 @@ template <> __device__ __forceinline__ double ex<double>(double x) { return exp(
 template <> __device__ __forceinline__ float ex<float>(float x) { return expf(x); }
 
 // exp(x) for |x| <= kSmallExp: minimax polynomial of (exp(x) - 1 - x) / x^2
-// (Remez exchange; relative error 3.4e-18 double, 3.1e-9 float before rounding,
-// largest error after it 1.2e-16 and 6.2e-8). No reduction and no scaling.
+// (Remez exchange; relative error with the rounded coefficients 1.4e-17 double,
+// 5.2e-9 float, largest error after rounding 1.2e-16 and 6.2e-8). No reduction
+// and no scaling.
 __device__ __forceinline__ double ex_poly(double x) {
   double p = 2.5117848056977748e-08;
   p = fma(p, x, 2.7631276855506471e-07);
@@ -165,11 +165,11 @@ template <bool IMAG, typename C> __device__ __forceinline__ C mul_phase(C p, C u
 // variants: inside one loop the compiler would evaluate the sin/cos or exp
 // of every alternative for every point and select afterwards.
 
-// The same with a non-temporal hint: every pass reads and writes each state
-// element exactly once, and streaming them past the caches shortens a pass
-// when a single instance leaves the chip mostly idle (for batched plans the
-// normal policy can be faster; the plan chooses, see the streaming flags of
-// sgpe_plan_set_streaming).
+// The same with a non-temporal hint, for the streaming flags of
+// sgpe_plan_set_streaming. The compiler merges the two arms of the passes'
+// run-time choice into one without the hint, so that the flags have no effect at
+// present (kept apart by force: 3 % of a 512^2 complex128 step gained, batched
+// 1024^2 complex64 70 % slower).
 template <typename C> __device__ __forceinline__ C ld_stream(const C* p) {
   typedef decltype(p->x) S;
   typedef S V2 __attribute__((ext_vector_type(2)));
@@ -1027,11 +1027,11 @@ __device__ __forceinline__ void row_item(const InstDev& P, typename Cx<R>::T* __
   // being held in registers since the loads and the inverse transform, which
   // compute the same addresses (held, they cost up to 70 VGPRs and spill the
   // 4096-point complex128 pass). It pays where registers are what limits
-  // the resident workgroups: 4096 points, and 1024-2048 points where the
-  // LDS admits three waves per SIMD (complex64 2048 points: 192 -> 130
-  // VGPRs, 58 -> 50 us per pass). Where the LDS allows two waves anyway
-  // (complex128 2048 points) or small batched rows, whose workgroups fill
-  // the CUs' slots already, only the recomputation remains (+2 %).
+  // the resident workgroups: 2048 points and more (complex64 2048 points: 192 ->
+  // 130 VGPRs, 58 -> 50 us per pass; complex128, unless HELD: 98 -> 79 us for 2048
+  // rows), and 1024 points where the LDS admits three waves per SIMD. With
+  // small batched rows, whose workgroups fill the CUs' slots already, only the
+  // recomputation remains (+2 %).
   constexpr size_t kLdsWg = kData * (kDb ? 2 : 1) + (kTw ? (size_t)N * sizeof(C) : 0);
   constexpr int kLdsWaves = (int)(kLdsBytes / kLdsWg) * ((ROWS * T + 63) / 64) / 4;
   constexpr bool kOpaque = HELD ? false : N >= 2048 || (N >= 1024 && kLdsWaves >= 3);

@@ -1,8 +1,11 @@
 // Split-step passes and standalone transforms for even lengths without a
-// compiled power-of-two kernel whose prime factors are at most 13 (32 to 2048
-// points; the rest stays with sgpe_generic.h).
+// compiled power-of-two kernel whose prime factors are at most 13, 32 to 2048
+// points. An inner stage has one butterfly per thread and a workgroup 512 threads:
+// columns and transforms of 1694, 1716, 1782, 2002 and 2028 points and rows (two
+// components at a time) of those and 1452, 1458, 1750, 1848, 1936, 1944 and 1980
+// have more and stay with sgpe_generic.h, as all other lengths do.
 //
-// A length is split on the host into two to five radices of at most 16
+// A length is split on the host into two to four radices of at most 16
 // (mix_factor). A stage is one register butterfly of compile-time radix per
 // work item (a uniform switch picks the radix); data pass between stages through
 // LDS. A pass runs
@@ -31,7 +34,7 @@
 
 namespace sgpe {
 
-constexpr int kMixMaxStages = 5;
+constexpr int kMixMaxStages = 4;
 constexpr int kMixMaxLen = 2048;
 constexpr int kMixMinLen = 32;
 constexpr int kMixMaxRadix = 16;

@@ -2,12 +2,13 @@
 
 For a grid length the library compiles several shapes of each pass: E
 elements per thread (the FFT's radix) and the number of rows (row pass) or
-columns (column pass) per workgroup; each pass can also stream its state
-accesses past the caches (non-temporal) or not. Which choice is fastest
-depends on the grid, the precision and how many instances share a launch
-(small single instances are latency-bound and want many small waves and
-streaming; large or batched ones want fewer, fatter threads). The tuner times
-every compiled shape in both cache modes with ``sgpe_profile_full_steps`` on
+columns (column pass) per workgroup; each pass also has a streaming flag
+(non-temporal state accesses or not), whose two values run the same code in
+the present build, so that what the table stores for it is noise. Which choice
+is fastest depends on the grid, the precision and how many instances share a
+launch (small single instances are latency-bound and want many small waves;
+large or batched ones want fewer, fatter threads). The tuner times every
+compiled shape in both cache modes with ``sgpe_profile_full_steps`` on
 a scratch plan (the caller's states are never touched), picks the fastest
 row and column choices independently and caches them in a JSON file keyed by
 precision, grid and batch-size bucket as

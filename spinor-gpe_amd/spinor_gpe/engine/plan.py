@@ -215,7 +215,8 @@ class Plan:
         return tuple(out)
 
     def set_streaming(self, row_stream, col_stream):
-        """Non-temporal (1) or normal (0) state accesses of each pass."""
+        """Non-temporal (1) or normal (0) state accesses of each pass (the same
+        instructions in the present build, see ``sgpe_plan_set_streaming``)."""
         self._call('sgpe_plan_set_streaming', int(bool(row_stream)), int(bool(col_stream)))
 
     def streaming(self):
