@@ -1038,6 +1038,19 @@ static void phase_host(double e_dt, bool imag, double* re, double* im) {
   }
 }
 
+// Whether |v[i]| h <= bound for all i (false for NaN); in blocks, so that an
+// array with large values is left early.
+static bool all_within(const double* v, size_t n, double h, double bound) {
+  const size_t block = 4096;
+  for (size_t i = 0; i < n; i += block) {
+    const size_t end = std::min(n, i + block);
+    int in = 1;
+    for (size_t j = i; j < end; ++j) in &= (int)(std::fabs(v[j]) * h <= bound);
+    if (!in) return false;
+  }
+  return true;
+}
+
 static int plan_load_slot(sgpe_plan* p, int slot, const sgpe_inst_desc* d, void* psik) {
   const int ny = p->ny, nx = p->nx, prec = p->prec;
   const size_t cs = csize(prec);
@@ -1074,6 +1087,14 @@ static int plan_load_slot(sgpe_plan* p, int slot, const sgpe_inst_desc* d, void*
   h.dt_sub[1] = dts[1];
   h.omega = d->coupling == SGPE_COUPLING_UNIFORM ? d->omega : 0.0;
   h.estride = 2 * nx + ny;
+  // Dense phases of the longer sub-step (the inner one).
+  const double bound = imag ? kSmallExp : kSmallAngle;
+  const size_t points = (size_t)ny * nx;
+  h.dense_small = 1;
+  for (int s = 0; s < 2; ++s)
+    if (d->v_dense[s] && h.dense_small) h.dense_small = all_within(d->v_dense[s], points, dts[1], bound);
+  if (d->coupling == SGPE_COUPLING_ARRAY && h.dense_small)
+    h.dense_small = all_within(d->omega_dense, points, 0.25 * dts[1], bound);
 
   Staging st;
   size_t o_kx[2][2], o_ky[2][2], o_px[2][2], o_py[2][2], o_eth = 0;

@@ -79,6 +79,7 @@ struct InstDev {
   int ny, nx;
   int imag;         // 1: imaginary time (t_step = -i dt), 0: real time
   int coupling;     // 0: none, 1: uniform Omega, 2: dense Omega array
+  int dense_small;  // 1: every phase V Delta, Omega Delta / 4 of the dense arrays is within kSmallAngle / kSmallExp
   double atom_num, g_uu, g_dd, g_ud;
   double dv_r, dv_k, fft_c;      // dx*dy, dkx*dky, dx*dy/(2 pi)
   double dt_sub[2];              // |sub-step| for DUR_OUT / DUR_IN

@@ -615,13 +615,14 @@ __device__ __forceinline__ void part_sums(const double* part, int nt2, int slot,
 //  - Where the phases of all points of a wave are small (they are g n dt / 2:
 //    about 1e-2), their sin/cos or exp is a polynomial alone; one wave-uniform
 //    test chooses the code for the whole block (SMALL). Tested per point, it
-//    would cut the block into pieces that cannot overlap.
+//    would cut the block into pieces that cannot overlap. Phases of dense
+//    potentials and couplings are judged once, on the host (dense_small).
 // Row pass before and after (dispatch times, us): 8 x 1024^2 complex64
 // imaginary time 75.5 -> 69.6, 16 x 512^2 complex64 imaginary 38.2 -> 35.6, one
 // 2048^2 complex128 real 86.9 -> 83.1, one 512^2 real 10.7 -> 10.2 (complex128)
 // and 7.9 -> 7.3 (complex64).
 template <typename R> struct RowCoef {
-  bool imag, theta;
+  bool imag, theta, dense_small;
   R kuu, kdd, kud;  // interaction phase of U per unnormalized density
   R sc;             // normalization x forward transform scale
   R ca, cb;         // a and b of C (b: its imaginary part in real time)
@@ -630,6 +631,7 @@ template <typename R> struct RowCoef {
     const double h = 0.5 * P.dt_sub[dur] * lam2;
     imag = P.imag != 0;
     theta = P.theta_x != nullptr;
+    dense_small = P.dense_small != 0;
     kuu = (R)(P.g_uu * h);
     kdd = (R)(P.g_dd * h);
     kud = (R)(P.g_ud * h);
@@ -682,15 +684,17 @@ template <int V> struct PointVariant { static constexpr int v = V; };
 // The theta-free variant is complex64's alone: there it saves 1-3 % of a batched
 // row pass, in complex128 the third way out of the branch costs more registers
 // than its arithmetic saves (32 x 256^2: 37.5 us with it, 32.3 without).
-template <typename R, class F>
+template <typename R, bool NT = sizeof(R) == 4, class F>
 __device__ __forceinline__ void with_variant(const RowCoef<R>& k, R top, F&& f) {
   if (k.imag) {
-    if (__builtin_amdgcn_ballot_w64(!(top <= (R)kSmallExp)))
+    if (__builtin_amdgcn_ballot_w64(!(top <= (R)kSmallExp))) {
       f(PointVariant<PV_IMAG>());
-    else if (sizeof(R) == 8 || k.theta)
+    } else {
+      if constexpr (NT) {
+        if (!k.theta) return f(PointVariant<PV_IMAG_SMALL_NT>());
+      }
       f(PointVariant<PV_IMAG_SMALL>());
-    else
-      f(PointVariant<PV_IMAG_SMALL_NT>());
+    }
   } else if (__builtin_amdgcn_ballot_w64(!(top <= (R)kSmallAngle))) {
     f(PointVariant<PV_REAL>());
   } else {
@@ -768,7 +772,13 @@ __device__ __forceinline__ R fast_top(const C (&a0)[E], const C (&a1)[E], const 
 }
 
 // Points J0 <= j < J1 of a row: FAST as above, else with dense potentials and
-// coupling arrays where the slot has them (point j at base + offset(j) of them).
+// coupling arrays where the slot has them (point j at base + offset(j) of
+// them). Their values are read inside the point loop: read ahead of the variant
+// test, for a test that counts them too, they cost 10 to 30 registers, which is a
+// wave per SIMD or a spill in most shapes. Row pass in imaginary time, dense
+// potential and coupling, us, read ahead -> here: 2048 x 1024 complex128 62.4 ->
+// 52.7, complex64 64.7 -> 43.9, 8 x 512^2 complex128 66.1 -> 57.6, complex64 35.4 ->
+// 33.2, one 512^2 complex128 12.8 -> 12.4.
 template <typename R, int E, bool FAST, int J0 = 0, int J1 = E, typename C, typename PY, typename At>
 __device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const InstDev& P, const RowCoef<R>& k,
                                               size_t base, const At& offset, const PY& py0, const PY& py1, const C (&tx0)[E],
@@ -778,42 +788,34 @@ __device__ __forceinline__ void row_pointwise(C (&a0)[E], C (&a1)[E], const Inst
       fast_points<R, decltype(v)::v, E, J0, J1>(a0, a1, k, py0, py1, tx0, tx1, tex);
     });
   } else {
-    constexpr int M = J1 - J0;
     const double* vd0 = P.v_dense[0];
     const double* vd1 = P.v_dense[1];
     const double* omd = P.coupling == 2 ? P.omega_dense : nullptr;
-    R v0[M], v1[M], an[M];
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-      const size_t at = base + offset(J0 + i);
-      v0[i] = vd0 ? (R)ld_global(vd0 + at) * k.dts : (R)0;
-      v1[i] = vd1 ? (R)ld_global(vd1 + at) * k.dts : (R)0;
-      an[i] = omd ? (R)ld_global(omd + at) * k.dts * (R)0.25 : (R)0;
-    }
-    R top = fast_top<R, E, J0, J1>(a0, a1, k);
-#pragma unroll
-    for (int i = 0; i < M; ++i) top = larger(larger(larger(top, v0[i]), v1[i]), an[i]);
-    with_variant<R>(k, top, [&](auto v) {
-      constexpr int V = decltype(v)::v == PV_IMAG_SMALL_NT ? PV_IMAG_SMALL : decltype(v)::v;
+    // A slot whose dense phases are not all small takes the general code; the
+    // interaction phases decide for the others.
+    const R top = k.dense_small ? fast_top<R, E, J0, J1>(a0, a1, k) : (R)INFINITY;
+    with_variant<R, false>(k, top, [&](auto v) {
+      constexpr int V = decltype(v)::v;
       constexpr bool IMAG = V >= PV_IMAG_SMALL_NT;
       constexpr bool SMALL = V != PV_REAL && V != PV_IMAG;
 #pragma unroll
-      for (int i = 0; i < M; ++i) {
-        const int j = J0 + i;
+      for (int j = J0; j < J1; ++j) {
+        const size_t at = base + offset(j);
         R a = k.ca, b = k.cb;
         if (omd) {
+          const R an = (R)ld_global(omd + at) * k.dts * (R)0.25;
           if constexpr (IMAG) {
-            const R g = SMALL ? ex_poly(an[i]) : ex<R>(an[i]), gi = (R)1 / g;
+            const R g = SMALL ? ex_poly(an) : ex<R>(an), gi = (R)1 / g;
             a = (R)0.5 * (g + gi);
             b = (R)-0.5 * (g - gi);
           } else {
-            const C u = phase_op<R, false, SMALL>(an[i]);
+            const C u = phase_op<R, false, SMALL>(an);
             a = u.x;
             b = u.y;
           }
         }
-        const C f0 = vd0 ? phase_op<R, IMAG, SMALL>(v0[i]) : pot_factor<IMAG>(tx0[j], py0[j]);
-        const C f1 = vd1 ? phase_op<R, IMAG, SMALL>(v1[i]) : pot_factor<IMAG>(tx1[j], py1[j]);
+        const C f0 = vd0 ? phase_op<R, IMAG, SMALL>((R)ld_global(vd0 + at) * k.dts) : pot_factor<IMAG>(tx0[j], py0[j]);
+        const C f1 = vd1 ? phase_op<R, IMAG, SMALL>((R)ld_global(vd1 + at) * k.dts) : pot_factor<IMAG>(tx1[j], py1[j]);
         R e0, e1;
         point_phases<R>(a0[j], a1[j], k, &e0, &e1);
         point_ops<R, V>(a0[j], a1[j], e0, e1, k.sc, a, b, f0, f1, tex[j]);
