@@ -1101,6 +1101,13 @@ static int plan_load_slot(sgpe_plan* p, int slot, const sgpe_inst_desc* d, void*
   size_t o_k2x[2][2][2], o_k2y[2][2][2];  // [previous][current duration][component]
   size_t o_tx[2], o_ty[2], o_vx[2], o_vy[2], o_thx = 0, o_td[2], o_vd[2], o_om = 0;
   const size_t dense = (size_t)ny * nx * sizeof(double);
+  // Room for everything below (with its alignment) at once: growing would copy
+  // the dense arrays, which come first.
+  size_t room = 64 * 256 + (size_t)(nx + ny) * (4 * sizeof(double) + 17 * cs) + nx * sizeof(double) +
+                (size_t)(PART_SLOTS * 2 * nx + EPART_SLOTS * (2 * nx + ny)) * sizeof(double);
+  for (int s = 0; s < 2; ++s) room += (d->t_dense[s] ? dense : 0) + (d->v_dense[s] ? dense : 0);
+  if (d->coupling == SGPE_COUPLING_ARRAY) room += dense;
+  st.bytes.reserve(room);
   for (int s = 0; s < 2; ++s) {
     o_tx[s] = o_ty[s] = o_vx[s] = o_vy[s] = o_td[s] = o_vd[s] = 0;
     if (d->t_dense[s]) {
