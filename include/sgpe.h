@@ -152,8 +152,8 @@ int sgpe_pops(sgpe_ctx* ctx, int precision, int ny, int nx, const void* psi0, co
  * requirement, pspinor.py:331-332), and powers of two up to 4096. Powers of
  * two from 64 up run on compiled register-FFT passes; other lengths (and a
  * power-of-two axis no compiled tile of which divides the other axis) on
- * runtime-length LDS mixed-radix passes, slower but with the same results
- * to rounding. Other sizes: SGPE_E_UNSUPPORTED. Slots start empty
+ * mixed-radix register passes or runtime-length LDS passes, slower but with the
+ * same results to rounding. Other sizes: SGPE_E_UNSUPPORTED. Slots start empty
  * and inactive; a plan can step once at least one slot is set (empty slots
  * are skipped), so a server can fill slots as requests arrive. */
 int sgpe_plan_create(sgpe_ctx* ctx, int precision, int ny, int nx, int n_slots, sgpe_plan** out);
@@ -212,8 +212,8 @@ int sgpe_plan_tune(sgpe_plan* plan, int row_e, int row_rows, int col_e, int col_
 int sgpe_list_shapes(int pass, int precision, int n, int* out_pairs, int cap);
 
 /* Current shapes: out4 = {row_e, row_rows, col_e, col_w}, negative row_rows
- * and col_w as in sgpe_plan_tune; row_e = 0 (col_e = 0): that pass runs on
- * the runtime-length kernels. */
+ * and col_w as in sgpe_plan_tune; row_e = 0 (col_e = 0): that pass runs
+ * without a compiled shape, on the mixed-radix or the runtime-length kernels. */
 int sgpe_plan_get_tuning(const sgpe_plan* plan, int* out4);
 
 /* Run blocks of full steps (sgpe_full_steps, sgpe_graph_steps, sgpe_group_run)

@@ -589,10 +589,10 @@ struct sgpe_plan {
   const KEntry* col = nullptr;
   const void* tw_x = nullptr;  // twiddles for nx (rows)
   const void* tw_y = nullptr;  // twiddles for ny (columns)
-  // Runtime-length kernels (sgpe_generic.h) of an axis without a compiled
-  // pass for its length or tiles: gen_x for the row pass (x transforms, row_e
-  // = 0, row_rows = 1), gen_y for the column pass (col_e = 0, col_w from
-  // gen_col_width); their stage radices and root tables.
+  // An axis without a compiled pass for its length or tiles: gen_x for the row
+  // pass (x transforms, row_e = 0, row_rows = 1), gen_y for the column pass
+  // (col_e = 0, col_w from mix_batch or gen_col_width); stage radices and root
+  // tables of the runtime-length kernels (sgpe_generic.h).
   bool gen_x = false, gen_y = false;
   // Column pass variant with its y phase tables in global memory (listed
   // with -W columns per block; col_w keeps the positive tile width).
@@ -639,7 +639,7 @@ static void drop_graphs(sgpe_plan* p) {
 }
 
 // Pass shapes of a plan. row_e = 0 (col_e = 0): the row (column) pass runs
-// on the runtime-length kernels, row_rows (col_w) then ignored.
+// without a compiled shape, row_rows (col_w) then ignored.
 static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col_w) {
   const bool gx = row_e == 0, gy = col_e == 0;
   if ((gx && !gen_length_ok(p->nx)) || (gy && !gen_length_ok(p->ny)))
@@ -647,7 +647,8 @@ static int plan_select(sgpe_plan* p, int row_e, int row_rows, int col_e, int col
   const size_t cs = csize(p->prec);
   // Without compiled passes: mixed-radix kernels where the length splits, else
   // the runtime-length ones. Tiles as wide as leaves two workgroups per CU;
-  // columns at least 64 bytes.
+  // columns at least 64 bytes where a divisor of nx, the LDS and the threads
+  // allow (1000 points, complex64: five columns, 40 bytes).
   MixFft mx{}, my{};
   int mrows = 0, mw = 0;
   if (gx) {
@@ -1394,7 +1395,8 @@ int sgpe_fft2(sgpe_ctx* ctx, int precision, int ny, int nx, int n_arrays, void* 
     int re, rr, ce, cw;
     default_row(precision, nx, &re, &rr);
     default_col(precision, ny, &ce, &cw);
-    // Compiled shapes where one fits, else the runtime-length kernels.
+    // Compiled shapes where one fits, else the mixed-radix or runtime-length
+    // kernels.
     const bool gx = !fit_shape(K_FROW, precision, nx, ny, &re, &rr);
     const bool gy = !fit_shape(K_FCOL, precision, ny, nx, &ce, &cw);
     if ((gx && !gen_length_ok(nx)) || (gy && !gen_length_ok(ny)))
@@ -1628,8 +1630,8 @@ int sgpe_plan_create(sgpe_ctx* ctx, int precision, int ny, int nx, int n_slots, 
     p->row_stream = p->col_stream = n_slots == 1 ? 1 : 0;
     p->h_inst.resize(n_slots);
     p->slots.resize(n_slots);
-    // Compiled default shapes where they fit the grid, else the runtime-length
-    // kernels for that axis (e = 0).
+    // Compiled default shapes where they fit the grid, else the mixed-radix or
+    // runtime-length kernels for that axis (e = 0).
     int re, rr, ce, cw;
     default_row_pass(precision, nx, (long)ny * n_slots, &re, &rr);
     default_col(precision, ny, &ce, &cw);

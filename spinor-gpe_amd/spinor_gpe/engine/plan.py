@@ -209,7 +209,8 @@ class Plan:
     def tuning(self):
         """(row E, rows per block, column E, columns per block); rows per
         block < 0: the split row layout with that many rows per block; E = 0:
-        that pass runs on the runtime-length kernels."""
+        that pass has no compiled shape (mixed-radix or runtime-length
+        kernels)."""
         out = (ctypes.c_int * 4)()
         nat.check(nat.lib().sgpe_plan_get_tuning(self.handle, out))
         return tuple(out)
